@@ -82,7 +82,8 @@ enum {
 /* factorisation modes */
 enum {
     STC_PLAIN_FP64 = 0,   /* complex128 LU with partial pivoting (zgetrf)      */
-    STC_REFINED_FP32 = 1  /* complex64 LU + FP64 iterative refinement        */
+    STC_REFINED_FP32 = 1  /* complex64 factors (LU, up to n = 128 the inverse),
+                             pivoted alike, + FP64 iterative refinement       */
 };
 
 typedef struct {
@@ -105,8 +106,9 @@ const char* stc_strerror(int code);
 int stc_device_ok(stc_handle h);
 
 /* ---- launch policy (set by an autotuner; optional) -----------------------------
- * How systems that do not fit the LDS whole are factored.  kernel: 0 =
- * automatic, 1 = 16-column register panel (three workgroups per CU for
+ * How systems are factored.  kernel: 0 = automatic (orders up to 128 in
+ * registers, except for stc_getrf and the refined adjoint; else the choices named
+ * below), 1 = 16-column register panel (three workgroups per CU for
  * complex64, two for complex128), 2 = wide panel held in LDS (16..64 columns,
  * one or two workgroups per CU, by lds_budget), 3 = as 2 with the trailing
  * update's complex products in Gauss 3M form (three real MFMA products instead
@@ -118,7 +120,8 @@ int stc_device_ok(stc_handle h);
  * workgroup, 0 = automatic, else 16384 .. 163584 (the LDS the panel may use
  * sets the workgroups per CU and the panel width).  jb_max: widest panel
  * (0 = no cap).  An entry applies to launches whose largest system has order
- * n in that mode, or the nearest order with an entry; NULL removes it.  The
+ * n in that mode, or the nearest order with an entry (launches up to order 128
+ * leave the registers only for an entry of such an order); NULL removes it.  The
  * results do not depend on the policy beyond rounding (pivots follow LAPACK
  * in every kernel).  No counterpart in the reference (its only tuning knob is a
  * fixed batch size, test/krylovMidsizeTest/gpu/concurrent/batchedLU/src/config/config.cu:29-30). */

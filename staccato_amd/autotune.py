@@ -1,6 +1,7 @@
 """Autotuner of the sweep kernel's launch policy, by measurement on the device.
 
-The blocked factorisation (systems that do not fit the LDS whole) can run as
+Systems up to n = 128 run in registers (the library's own choice), larger ones
+by a blocked factorisation; either can also run as
   - the 16-column register panel (kernel 1: three workgroups per CU for
     complex64, two for complex128), or
   - the wide LDS panel (kernel 2) with 160 KiB of LDS per workgroup (one per
@@ -41,6 +42,8 @@ CANDIDATES = [
     # Gauss 3M complex products in the trailing update (complex64 only)
     ("wide-3M-2perCU", 3, 80 * 1024, 0),
     ("wide-3M-1perCU", 3, 160 * 1024 - 256, 0),
+    # the library's own choice (up to n = 128: systems in registers)
+    ("automatic", 0, 0, 0),
 ]
 
 
@@ -92,7 +95,7 @@ def apply_cached(handle, n, nrhs, mode, cache=None):
 def automatic_name(n, mode):
     complex64 = mode in ("refined", "fp32", 1)
     if n <= 128:
-        return "register-panel"
+        return "automatic"
     one_per_cu = n > (512 if complex64 else 256)
     if n > 256:  # the two-level update (complex128 beyond n = 512: register panel either way)
         return "wide-2level-1perCU" if one_per_cu else "wide-2level-2perCU"

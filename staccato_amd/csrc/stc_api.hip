@@ -108,7 +108,7 @@ struct stc_ctx {
     int live_plans = 0;
     std::map<std::pair<int, int>, Policy> policy;  // (order n, refine) -> policy
     // staging for host-memory calls
-    DevBuf freq, F, X, info, berr, iters, fac, ipiv, sys, items, adj, c, phi, kd, A, load;
+    DevBuf freq, F, X, info, berr, iters, fac, ipiv, sys, items, adj, c, phi, phiT, kd, A, load;
 };
 
 struct stc_plan_s {
@@ -263,17 +263,50 @@ Policy policy_for(const stc_ctx* h, int n, int refine) {
 struct LaunchCfg {
     int refine = 0;
     int maxr = 1;
-    int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path, 2 with 3M products, 3 two-level
+    int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path, 2 with 3M products, 3 two-level;
+                    // reg_kernel: 4, with the adjoint 5
+    int threads = kThreads;
     int lds = 0;
     int grid = 1;
     size_t slot_elems = 0;
     size_t slot_bytes = 0;  // bytes of one factor slot (0: no blocked system)
 };
 
+constexpr int kKindReg = 4, kKindRegAdj = 5;
+
+// Systems that reg_kernel solves in registers: every order up to 128, unless
+// the factors themselves are asked for, the adjoint is refined (it needs the
+// inverse's transpose), or a policy set for an order in that range names
+// another kernel.  Faster than the kernels it replaces at every order measured (the
+// figures are at reg_kernel); above 128 the matrix does not fit the registers of one
+// workgroup with room to work.
+bool use_registers(const stc_ctx* h, int maxn, int refine, int adj, int fac) {
+    if (maxn > kRegMaxN || fac || (refine && adj)) return false;
+    const Policy* p = nullptr;
+    int bd = 0x7fffffff;
+    for (const auto& kv : h->policy)
+        if (kv.first.second == refine && kv.first.first <= kRegMaxN && std::abs(kv.first.first - maxn) < bd) {
+            bd = std::abs(kv.first.first - maxn);
+            p = &kv.second;
+        }
+    return !p || (p->kernel == 0 && p->lds_budget == 0 && p->jb_max == 0);
+}
+
+// Workgroups of the launch that fit one CU.
+int resident(const LaunchCfg* cfg, int* per_cu) {
+    void* kfun = sweep_kernel_fn(cfg->refine, cfg->maxr, cfg->wide);
+    if (!kfun) return STC_EINVAL;
+    HIP_TRY(hipFuncSetAttribute(kfun, hipFuncAttributeMaxDynamicSharedMemorySize, cfg->lds));
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, kfun, cfg->threads, cfg->lds));
+    if (*per_cu < 1) *per_cu = 1;
+    return STC_OK;
+}
+
 // Layout and grid of a launch, no allocation (host or device): grid = resident
 // workgroups, capped by the points and, when slot_budget > 0, by the factor
 // slots that fit in slot_budget bytes (STC_ETOOBIG when not even one does).
-int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine, int adj,
+// fac: the factors are asked for (stc_getrf).
+int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine, int adj, int fac,
                 size_t slot_budget, LaunchCfg* cfg) {
     const int ts = refine ? 8 : 16;
     int maxn = 0;
@@ -284,6 +317,19 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
     cfg->refine = refine;
     cfg->maxr = maxr;
     const Policy pol = policy_for(h, maxn, refine);
+    if (use_registers(h, maxn, refine, adj, fac)) {
+        cfg->wide = adj ? kKindRegAdj : kKindReg;
+        cfg->threads = 64 * reg_waves(refine, maxr);
+        cfg->lds = 0;
+        for (int i = 0; i < nsys; ++i)
+            cfg->lds = std::max(cfg->lds, refine ? reg_lds_refined(sys[i].n)
+                                                 : reg_lds_plain(sys[i].n, reg_waves(refine, maxr), adj));
+        int per_cu = 0;
+        const int rc = resident(cfg, &per_cu);
+        if (rc) return rc;
+        cfg->grid = (int)std::max(1LL, std::min((long long)h->num_cu * per_cu, nitems));
+        return STC_OK;
+    }
     // the register-resident panel holds 4 (or 2, 1) columns per wavefront
     int jb_cap = kWaves * panel_cols_per_wave(ts, maxr);
     if (pol.jb_max > 0) jb_cap = std::max(4, std::min(pol.jb_max, jb_cap));
@@ -320,12 +366,8 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
             cfg->lds = lds;
         }
     }
-    void* kfun = sweep_kernel_fn(refine, maxr, cfg->wide);
-    if (!kfun) return STC_EINVAL;
-    HIP_TRY(hipFuncSetAttribute(kfun, hipFuncAttributeMaxDynamicSharedMemorySize, cfg->lds));
     int per_cu = 0;
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfun, kThreads, cfg->lds));
-    if (per_cu < 1) per_cu = 1;
+    if ((rc = resident(cfg, &per_cu))) return rc;
     long long g = (long long)h->num_cu * per_cu;
     // every blocked system factors in a per-workgroup slot (also for stc_getrf,
     // which copies the slot out in LAPACK layout afterwards)
@@ -356,8 +398,11 @@ int enqueue_raw(const LaunchCfg& cfg, KParams& kp, int* counter, void* scratch, 
     kp.scratch = scratch;
     kp.slot_elems = cfg.slot_elems;
     kp.lds_budget = cfg.lds;
-    hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, st, kp.counter);
-    HIP_TRY(hipGetLastError());
+    // the register kernel deals the points of a single system out by itself
+    if (cfg.wide < kKindReg || kp.items) {
+        hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(64), 0, st, kp.counter);
+        HIP_TRY(hipGetLastError());
+    }
     HIP_TRY(sweep_kernel_launch(cfg.refine, cfg.maxr, cfg.wide, cfg.grid, cfg.lds, st, kp));
     return STC_OK;
 }
@@ -365,8 +410,8 @@ int enqueue_raw(const LaunchCfg& cfg, KParams& kp, int* counter, void* scratch, 
 // Plan a launch and size the handle's factor slots for it.  Growing the slots
 // frees the old ones, so the handle's previous launch is waited for first.
 int configure(stc_ctx* h, std::vector<SysDesc>& sys, long long nitems, int refine, int adj,
-              LaunchCfg* cfg) {
-    int rc = plan_launch(h, sys.data(), (int)sys.size(), nitems, refine, adj, 0, cfg);
+              LaunchCfg* cfg, int fac = 0) {
+    int rc = plan_launch(h, sys.data(), (int)sys.size(), nitems, refine, adj, fac, 0, cfg);
     if (rc) return rc;
     const size_t need = cfg->slot_bytes * (size_t)cfg->grid;
     if (need > h->scratch.bytes) {
@@ -461,6 +506,12 @@ __global__ void load_rhs_kernel(const double2* B, int n, int nin, const double2*
     F[e] = make_double2(re, im);
 }
 
+// T (p x n, ld p) = transpose of A (n x p, ld n)
+__global__ void transpose_kernel(const double* A, int n, int p, double* T) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < n * p) T[e] = A[e / p + (size_t)(e % p) * n];
+}
+
 }  // namespace
 
 // ============================================================================
@@ -529,7 +580,7 @@ int stc_destroy(stc_handle h) {
         }
         DevBuf* bufs[] = {&h->scratch, &h->counter, &h->freq, &h->F, &h->X, &h->info, &h->berr,
                           &h->iters, &h->fac, &h->ipiv, &h->sys, &h->items, &h->adj, &h->c,
-                          &h->phi, &h->kd, &h->A, &h->load};
+                          &h->phi, &h->phiT, &h->kd, &h->A, &h->load};
         for (DevBuf* b : bufs) b->release();
         (void)hipStreamDestroy(h->stream);
     }
@@ -704,7 +755,7 @@ int stc_sweep_dev_noalloc(stc_handle h, int rom_id, int nfreq, const double* d_f
     s.info = d_info;
     s.berr = d_berr;
     LaunchCfg cfg;
-    int rc = plan_launch(h, &s, 1, nfreq, mode == STC_REFINED_FP32, 0, kNoAllocBytes - kNoAllocHead, &cfg);
+    int rc = plan_launch(h, &s, 1, nfreq, mode == STC_REFINED_FP32, 0, 0, kNoAllocBytes - kNoAllocHead, &cfg);
     if (rc) return rc;
     kp.one = s;
     kp.nitems = nfreq;
@@ -817,7 +868,7 @@ int stc_getrf(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int mo
     s.factor_out = h->fac.p;
     s.ipiv_out = h->ipiv.as<int>();
     LaunchCfg cfg;
-    rc = configure(h, sys, nfreq, refine, 0, &cfg);
+    rc = configure(h, sys, nfreq, refine, 0, &cfg, 1);
     if (rc) return rc;
     kp.one = sys[0];
     kp.nitems = nfreq;
@@ -991,7 +1042,7 @@ int stc_plan_create(stc_handle h, int nsys, const stc_sys_desc* dev_sys, int mod
     if (items.empty()) return STC_EINVAL;
     const bool refine = mode == STC_REFINED_FP32;
     LaunchCfg cfg;
-    if ((rc = plan_launch(h, sys.data(), (int)sys.size(), (long long)items.size(), refine, 0, 0, &cfg)))
+    if ((rc = plan_launch(h, sys.data(), (int)sys.size(), (long long)items.size(), refine, 0, 0, 0, &cfg)))
         return rc;
     stc_plan_s* p = new stc_plan_s();
     p->h = h;
@@ -1118,6 +1169,14 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     const bool refine = mode == STC_REFINED_FP32;
     LaunchCfg cfg;
     if ((rc = configure(h, sys, nfreq, refine, 1, &cfg))) return rc;
+    if (cfg.wide == kKindRegAdj) {  // reads Phi along its modes
+        if ((rc = h->phiT.ensure(ph.size() * sizeof(double)))) return rc;
+        const int cnt = n * std::max(p, 1);
+        hipLaunchKernelGGL(transpose_kernel, dim3((cnt + 255) / 256), dim3(256), 0, st, h->phi.as<double>(), n,
+                           std::max(p, 1), h->phiT.as<double>());
+        HIP_TRY(hipGetLastError());
+        sys[0].PhiT = h->phiT.as<double>();
+    }
     kp.one = sys[0];
     kp.nitems = nfreq;
     if ((rc = enqueue(h, cfg, kp, st))) return rc;

@@ -52,6 +52,7 @@ struct SysDesc {
     // adjoint
     const double2* c;    // n
     const double* Phi;   // n x p, ld = n
+    const double* PhiT;  // p x n, ld = p (register kernel)
     const double* kdiag; // p
     double* adj_out;     // nfreq blocks of (p + 2): J_w, dJ/deta_w, dJ/ds_k,w
     // fused output projection: C nout x n (ld nout), Y nfreq blocks of
@@ -253,6 +254,31 @@ inline Layout plan_layout_wide(int n, int nrhs, int ts, int budget, int jb_cap, 
     }
     L.lds = 0x7fffffff;
     return L;
+}
+
+// ---- register-resident systems (reg_kernel, n <= 128) ----------------------------------
+constexpr int kRegMaxN = 128;
+// Wavefronts per workgroup: four, and eight for complex128 above n = 64 (a
+// 128 x 128 complex128 matrix is 128 registers a lane on eight wavefronts).
+__host__ __device__ constexpr int reg_waves(int refine, int maxr) { return !refine && maxr == 2 ? 8 : 4; }
+
+// Dynamic LDS of reg_point_refined for order n.
+// multiplier columns, positions, scalars, pivots, xs (4 solutions), parts (the wavefronts'
+// partial sums of the residual or of a correction), rv (scaled residuals).
+__host__ __device__ inline int reg_lds_refined(int n) {
+    return align16((n <= 64 ? 12LL : 8LL) * n * 8) + align16(n * 4LL) + 64 + align16(n * 8LL) + align16(16 * 8) + align16(4LL * n * 16) +
+           align16(4LL * 4 * n * 16) + align16(4LL * n * 8);
+}
+
+// Dynamic LDS of reg_point_plain.
+// Scalars, reciprocals of the pivots, positions, multiplier columns (later one
+// vector per wavefront), two vectors and sums for the adjoint, U (or L) packed.
+__host__ __device__ inline int reg_packed_bytes(int n, int nw, int adj) {
+    const int u = 16 * (n * (n + 1) / 2), m = adj ? nw * 4 * 64 * 8 : 0;  // adjoint: also the modal partial sums
+    return u > m ? u : m;
+}
+__host__ __device__ inline int reg_lds_plain(int n, int nw, int adj) {
+    return 64 + 16 * n + align16(n * 4LL) + 16 * (nw == 8 ? 12 : 8) * n + (adj ? 32 * n + 2 * nw * 8 : 0) + reg_packed_bytes(n, nw, adj);
 }
 
 }  // namespace stc

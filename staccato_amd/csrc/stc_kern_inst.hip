@@ -13,7 +13,7 @@
 #error "STC_INST_MAXR (1, 2, 4, 8 or 16) must be defined"
 #endif
 #ifndef STC_INST_WIDE
-#error "STC_INST_WIDE (0: register panel, 1: wide panel, 2: wide panel with 3M products, 3: wide panel with the two-level update) must be defined"
+#error "STC_INST_WIDE (0: register panel, 1: wide panel, 2: wide panel with 3M products, 3: wide panel with the two-level update, 4: register-resident systems, 5: the same with the adjoint) must be defined"
 #endif
 
 #define STC_CAT2(a, b, c, d) a##b##_##c##_##d
@@ -25,11 +25,18 @@ namespace stc {
 
 using InstT = typename std::conditional<STC_INST_REFINE != 0, float, double>::type;
 
-void* STC_FN_PTR() { return reinterpret_cast<void*>(&sweep_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE>); }
+#if STC_INST_WIDE >= 4
+#define STC_KERNEL reg_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE == 5>
+constexpr int kInstThreads = 64 * reg_waves(STC_INST_REFINE, STC_INST_MAXR);
+#else
+#define STC_KERNEL sweep_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE>
+constexpr int kInstThreads = kThreads;
+#endif
+
+void* STC_FN_PTR() { return reinterpret_cast<void*>(&STC_KERNEL); }
 
 hipError_t STC_FN_LAUNCH(int grid, int lds, hipStream_t st, const KParams& kp) {
-    hipLaunchKernelGGL((sweep_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE>), dim3(grid), dim3(kThreads), lds,
-                       st, kp);
+    hipLaunchKernelGGL((STC_KERNEL), dim3(grid), dim3(kInstThreads), lds, st, kp);
     return hipGetLastError();
 }
 

@@ -1623,11 +1623,13 @@ namespace stc {
 // nout x n matrix C (ld nout).  Many outputs: one per thread, the reads of C
 // coalesced over o.  Few outputs (nout << n): one per wavefront, its lanes
 // split the sum over i and reduce by butterfly.  Only Y leaves the workgroup.
+// NT: threads of the workgroup.
+template <int NT = kThreads>
 __device__ __forceinline__ void project_cols(const SysDesc& s, int fidx, const z64* xs, int g0, int gc) {
     const int n = s.n, nout = s.nout, tid = threadIdx.x, q = nout * gc;
     double2* Y = s.Y + ((size_t)fidx * s.nrhs + g0) * nout;
-    if (q >= kThreads / 2) {
-        for (int e = tid; e < q; e += kThreads) {
+    if (q >= NT / 2) {
+        for (int e = tid; e < q; e += NT) {
             const int o = e % nout;
             const z64* x = xs + (size_t)(e / nout) * n;
             double re = 0.0, im = 0.0;
@@ -1641,7 +1643,7 @@ __device__ __forceinline__ void project_cols(const SysDesc& s, int fidx, const z
         }
     } else {
         const int lane = tid & 63;
-        for (int e = tid >> 6; e < q; e += kWaves) {
+        for (int e = tid >> 6; e < q; e += NT / 64) {
             const int o = e % nout;
             const z64* x = xs + (size_t)(e / nout) * n;
             double re = 0.0, im = 0.0;
@@ -1904,3 +1906,5 @@ sweep_kernel(KParams kp) {
 }
 
 }  // namespace stc
+
+#include "stc_reg.h"
