@@ -366,6 +366,7 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
             cfg->lds = lds;
         }
     }
+    cfg->threads = sweep_threads(refine, maxr, cfg->wide);
     int per_cu = 0;
     if ((rc = resident(cfg, &per_cu))) return rc;
     long long g = (long long)h->num_cu * per_cu;

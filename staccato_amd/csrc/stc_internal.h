@@ -12,12 +12,26 @@
 
 namespace stc {
 
-constexpr int kThreads = 256;   // 4 wavefronts of 64 lanes per workgroup
+// Threads per workgroup of sweep_kernel: four wavefronts, and eight in the wide-panel
+// kernels whose LDS panel leaves room for one workgroup per CU only (complex64 above
+// n = 512, complex128 above n = 256).  They keep all eight wavefronts that the
+// registers allow busy: with four, every latency of the trailing update and the residuals
+// was exposed (512 points: n = 1024 refined, 16 right-hand sides 108.4 -> 64.4 ms;
+// n = 512 plain, 4 right-hand sides 12.3 -> 11.0 ms).
+__host__ __device__ constexpr int sweep_threads(int refine, int maxr, int wide) {
+    return wide >= 1 && wide <= 3 && maxr >= (refine ? 16 : 8) ? 512 : 256;
+}
+#ifdef STC_INST_WIDE
+constexpr int kThreads = sweep_threads(STC_INST_REFINE, STC_INST_MAXR, STC_INST_WIDE);
+#else
+constexpr int kThreads = 256;
+#endif
 constexpr int kWaves = kThreads / 64;
+constexpr int kMaxWaves = 8;    // what the LDS layouts allow for
 constexpr int kMaxGroup = 4;    // right-hand sides solved together
 constexpr int kRedSlots = 1 + 5 * kMaxGroup;  // block reductions in the residual
 // reduction scratch: one row of kRedSlots per wave, the result row, scale factors
-constexpr int kRedDoubles = (kWaves + 1) * kRedSlots + kMaxGroup;
+constexpr int kRedDoubles = (kMaxWaves + 1) * kRedSlots + kMaxGroup;
 
 // flags of a launch
 enum : int {
@@ -206,7 +220,7 @@ __host__ __device__ constexpr int wide_jb_max(int elem_bytes) { return elem_byte
 // 16 x 16 diagonal blocks, the sub-panel's two alternating pivot-candidate
 // buffers (per wave one row of 16 and its 16-byte key) and the moved-row
 // list (2 x 16).  maxr is not needed (kept for the callers' signature).
-__host__ __device__ inline long long wide_cand_bytes(int ts) { return 2LL * kWaves * kSB * ts + 2LL * kWaves * 16; }
+__host__ __device__ inline long long wide_cand_bytes(int ts) { return 2LL * kMaxWaves * kSB * ts + 2LL * kMaxWaves * 16; }
 __host__ __device__ inline long long wide_lds_bytes(int n, int jb, int ts, int maxr) {
     (void)maxr;
     return align16((long long)(n | 1) * jb * ts) + align16((long long)jb * kSB * ts) + align16(wide_cand_bytes(ts)) +

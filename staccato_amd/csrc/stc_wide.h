@@ -206,7 +206,7 @@ __device__ __forceinline__ void subpanel_moves(cx<T>* __restrict__ P, int ldp, i
 template <typename T, int MAXR>
 __device__ __forceinline__ void subpanel_factor(cx<T>* __restrict__ P, int m, int ldp, int jbl, int c0, int sbw, int j0,
                                                 int* ipiv, int* rmap, int* sc, cx<T>* rowbuf, int2* mvl) {
-    constexpr int RM = MAXR >= 4 ? MAXR / 4 : 1;  // rows per thread
+    constexpr int RM = (64 * MAXR + kThreads - 1) / kThreads;  // rows per thread
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int mq = m - c0;
     cx<T>* Q = P + c0 + (size_t)c0 * ldp;  // sub-panel origin, ld ldp
@@ -581,8 +581,9 @@ __device__ __forceinline__ void subpanel_factor_1w(cx<float>* __restrict__ P, in
 template <typename T>
 __device__ __forceinline__ void invert_unit_lower16(const cx<T>* Q, int ldq, int kb, cx<T>* Linv,
                                                     cx<T>* __restrict__ Lg) {
-    static_assert(kThreads == kSB * kSB, "one thread per entry of the block");
+    static_assert(kThreads >= kSB * kSB, "one thread per entry of the block");
     const int tid = threadIdx.x;
+    if (kThreads > kSB * kSB && tid >= kSB * kSB) return;
     const int i = tid & 15, c = tid >> 4;  // thread (i, c) holds X[i][c]
     cx<T> lrow[kSB - 1];                   // L[i][k] for k < i (zero for rows >= kb)
 #pragma unroll
