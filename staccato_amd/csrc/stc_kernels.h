@@ -122,17 +122,22 @@ __device__ __forceinline__ void cfma(cx<T>& acc, cx<T> a, cx<T> b) {
     acc.im = fma(a.re, b.im, acc.im);
     acc.im = fma(a.im, b.re, acc.im);
 }
-// 1 / z by Smith's method (no overflow of |z|^2)
+// 1 / z without overflow of |z|^2
 template <typename T>
-__device__ __forceinline__ cx<T> crecip(cx<T> z) {
-    if (fabs(z.re) >= fabs(z.im)) {
-        T r = z.im / z.re;
-        T d = z.re + z.im * r;
-        return cmk<T>(T(1) / d, -r / d);
-    }
-    T r = z.re / z.im;
-    T d = z.im + z.re * r;
-    return cmk<T>(r / d, T(-1) / d);
+__device__ __forceinline__ cx<T> crecip(cx<T> z);
+// 1 / z, complex128: z scaled by a power of two to [1, 2) in its larger part,
+// one reciprocal of |z|^2 (hardware estimate and two Newton steps).  Smith's
+// form takes three divisions in a chain; same error (2 ulp against 2.5).
+template <>
+__device__ __forceinline__ cx<double> crecip(cx<double> z) {
+    const double a = fabs(z.re) >= fabs(z.im) ? z.re : z.im;
+    const int e = -__builtin_amdgcn_frexp_exp(a);
+    const double x = __builtin_amdgcn_ldexp(z.re, e), y = __builtin_amdgcn_ldexp(z.im, e);
+    const double q = fma(x, x, y * y);
+    double r = __builtin_amdgcn_rcp(q);
+    r = fma(fma(-q, r, 1.0), r, r);
+    r = fma(fma(-q, r, 1.0), r, r);
+    return cmk<double>(__builtin_amdgcn_ldexp(x * r, e), __builtin_amdgcn_ldexp(-y * r, e));
 }
 // complex64 (the factor of the refined mode, whose rounding the FP64
 // refinement absorbs): Smith's scaling with one hardware reciprocal
@@ -198,11 +203,20 @@ __device__ __forceinline__ z64 ld_z(const double2* p) {
 __device__ __forceinline__ void st_z(double2* p, z64 a) { *p = make_double2(a.re, a.im); }
 // NaN-propagating max
 __device__ __forceinline__ double nmax(double a, double b) { return (a > b || a != a) ? a : b; }
-// |a| for norms: sqrt(re^2 + im^2), falling back to hypot's scaling only
-// when the squares overflow or underflow
+// |a| for norms, scaled by a power of two so that the squares stay in range:
+// an estimate of 1 / sqrt and two Newton steps (1 ulp); infinite when a part is
 __device__ __forceinline__ double zabs(z64 a) {
-    const double q = fma(a.re, a.re, a.im * a.im);
-    return (q < 1e300 && q > 1e-300) || q == 0.0 ? sqrt(q) : hypot(a.re, a.im);
+    const double m = __builtin_fmax(fabs(a.re), fabs(a.im));
+    const int e = __builtin_amdgcn_frexp_exp(m);
+    const double x = __builtin_amdgcn_ldexp(a.re, -e), y = __builtin_amdgcn_ldexp(a.im, -e);
+    const double q = fma(x, x, y * y);
+    const double y0 = __builtin_amdgcn_rsq(q);
+    double h = 0.5 * y0, g = q * y0;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, q), h, g);
+    return q == 0.0 || m == __builtin_inf() ? m : __builtin_amdgcn_ldexp(g, e);
 }
 
 // ---- assembly: element e (column-major, ld = n) of A(w) in FP64 ---------------
@@ -219,6 +233,37 @@ __device__ __forceinline__ z64 assemble_at(const SysDesc& s, size_t e, double w,
     if (s.has_D) d = ldc<1>(reinterpret_cast<const z64*>(s.D) + e);
     return cmk<double>(k.re - s.eta * k.im - w2 * m.re - w * d.im,
                        k.im + s.eta * k.re - w2 * m.im + w * d.re);
+}
+
+// ---- operator kinds of the assembly (uniform per point) ------------------------------------------
+// The kind is decided around a batch of entries: its branches around each entry would make
+// every load of the batch wait by itself.
+enum : int { kOpReal2 = 0, kOpReal3 = 1, kOpCplx = 2 };
+__device__ __forceinline__ int op_kind(const SysDesc& s) {
+    return s.real_ops ? (s.has_D ? kOpReal3 : kOpReal2) : kOpCplx;
+}
+// f(integral_constant<kind>) for the point's kind
+template <typename F>
+__device__ __forceinline__ void with_kind(const SysDesc& s, F&& f) {
+    const int k = op_kind(s);
+    if (k == kOpReal2) f(std::integral_constant<int, kOpReal2>{});
+    else if (k == kOpReal3) f(std::integral_constant<int, kOpReal3>{});
+    else f(std::integral_constant<int, kOpCplx>{});
+}
+// Entry e of A(w), as assemble_at; explicit matrices (op_stride) read the
+// matrix once (M aliases K there).
+template <int KIND>
+__device__ __forceinline__ z64 elem_at(const SysDesc& s, size_t e, double w, double w2) {
+    if (KIND == kOpReal2 || KIND == kOpReal3) {
+        const double k = lds1<1>(s.K + e), m = lds1<1>(s.M + e);
+        const double d = KIND == kOpReal3 ? lds1<1>(s.D + e) : 0.0;
+        return cmk<double>(k - w2 * m, s.eta * k + w * d);
+    }
+    const z64 k = ldc<1>(reinterpret_cast<const z64*>(s.K) + e);
+    z64 m = k, d = czero<double>();
+    if (!s.op_stride) m = ldc<1>(reinterpret_cast<const z64*>(s.M) + e);
+    if (s.has_D) d = ldc<1>(reinterpret_cast<const z64*>(s.D) + e);
+    return cmk<double>(k.re - s.eta * k.im - w2 * m.re - w * d.im, k.im + s.eta * k.re - w2 * m.im + w * d.re);
 }
 
 // ---- pivot key of a candidate row: |re| + |im|, with LAPACK izamax's NaN rule ------
@@ -368,12 +413,7 @@ struct Mfma<double> {
 };
 
 constexpr int kSolveBlock = 32; // diagonal block of the blocked triangular solves
-// Operator columns per load round of the residual: 8 in the complex64 kernel
-// (168 registers per lane), 16 in the complex128 one (256).
-template <typename T>
-struct ResCols {
-    static constexpr int K = sizeof(T) == 4 ? 8 : 16;
-};
+constexpr int kResRows = 4;     // rows per lane of the residual
 constexpr int kUw = kUwCols;    // columns of one wave's U12 chunk
 constexpr int kUwLd = kUwLdCols;
 
@@ -1174,12 +1214,14 @@ __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* 
             for (int g = wave; g < gc; g += kWaves) {
                 cx<T>* y = w + (size_t)g * n + k0;
                 cx<T> v = lane < kb ? ldc<3>(y + lane) : czero<T>();
+                cx<T> rd = czero<T>();  // reciprocal of this lane's diagonal entry
+                if (!UNIT) {
+                    const cx<T> d = ldc<3>(Dg + min(lane, kb - 1) * (B + 1));
+                    rd = crecip(CONJ ? cconj(d) : d);
+                }
                 if (FWD) {
                     for (int k = 0; k < kb; ++k) {
-                        if (!UNIT && lane == k) {
-                            const cx<T> d = ldc<3>(Dg + (k + k * B));
-                            v = cdiv(v, CONJ ? cconj(d) : d);
-                        }
+                        if (!UNIT && lane == k) v = cmul(v, rd);
                         const cx<T> vk = cbcast(v, k);
                         if (lane > k && lane < kb) {
                             const cx<T> a = TRANS ? ldc<3>(Dg + (k + lane * B)) : ldc<3>(Dg + (lane + k * B));
@@ -1188,10 +1230,7 @@ __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* 
                     }
                 } else {
                     for (int k = kb - 1; k >= 0; --k) {
-                        if (!UNIT && lane == k) {
-                            const cx<T> d = ldc<3>(Dg + (k + k * B));
-                            v = cdiv(v, CONJ ? cconj(d) : d);
-                        }
+                        if (!UNIT && lane == k) v = cmul(v, rd);
                         const cx<T> vk = cbcast(v, k);
                         if (lane < k) {
                             const cx<T> a = TRANS ? ldc<3>(Dg + (k + lane * B)) : ldc<3>(Dg + (lane + k * B));
@@ -1299,100 +1338,169 @@ __device__ void block_sum(double (&vals)[NS], double* red) {
 // need_anorm), then per column g: out[1+4g] = ||r||_inf, out[2+4g] = ||x||_inf,
 // out[3+4g] = ||b||_inf, out[4+4g] = max |re r| + |im r|.
 // b is global (ldb) when bg != nullptr, else LDS (bl, ld n).
-// BF: the real-operator rounds without branches (columns beyond n contribute
-// zero, right-hand sides g >= gc repeat column gc - 1 and are discarded), so
-// the compiler interleaves a round's loads with its arithmetic; it needs more
-// registers and is used by the complex64 wide-panel kernel only.
-// RG: rs may be global memory (generic stores), else it is LDS.
-template <bool ADJ, int RC, bool BF, bool RG = false>
-__device__ __forceinline__ void residual(const SysDesc& s, double w, double w2, const double2* bg, int ldb,
-                         const z64* bl, const z64* xs, z64* rs, int gc, bool need_anorm,
-                         double* red, double (&out)[kRedSlots]) {
-    const int n = __builtin_amdgcn_readfirstlane(s.n), tid = threadIdx.x;
-    gc = __builtin_amdgcn_readfirstlane(gc);
-    // pass 1: r = b - op(A) x (and the row sums of |op(A)|), RC columns of
-    // the operators in flight per round
-    double amax = 0.0;
-    for (int i = tid; i < n; i += kThreads) {
-        z64 acc[kMaxGroup];
+// RG: rs may be global memory (generic accesses), else it is LDS.  sc: scratch, n * gc * ts
+// bytes of LDS (the free solve vectors).
+//
+// A pass over the operators (from the caches, 24 bytes a real entry) for gc solutions that
+// lie in LDS.  Every wavefront takes kResRows rows a lane and its share of the columns: a
+// solution entry is then read from LDS once for 4 * 64 rows (that read, 16 bytes for each
+// wavefront, column and right-hand side, bounded one row a lane), and the loops over the
+// rows and right-hand sides have no branch (columns g >= gc repeat column gc - 1), so that
+// the reads of a column batch are in flight together; real operators are loaded a batch
+// ahead.  The wavefronts' partial sums are added one wavefront after the other.  ADJ, whose
+// lanes stand n entries apart, takes one row a lane, all columns and eight of them (one
+// 64-byte piece a lane) per batch.  RC: columns of a batch.  With one
+// row a lane and a branch per right-hand side a pass took 148k cycles at n = 256 (two
+// workgroups per CU, refined, 4 right-hand sides) and 97k at n = 144, 112k and 72k now.
+template <bool ADJ, bool RG, int NG, int RC>
+__device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double w2, const double2* bg, int ldb,
+                              const z64* bl, const z64* xs, z64* rs, int gc, bool need_anorm,
+                              char* sc, int sc_bytes, double& amax) {
+    constexpr int NR = ADJ ? 1 : kResRows, NS = ADJ ? 1 : kWaves;  // NS: shares of the columns
+    const int n = __builtin_amdgcn_readfirstlane(s.n), tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int clo = ADJ ? 0 : wave * n / kWaves, chi = ADJ ? n : (wave + 1) * n / kWaves;
+    // the running sums of a row block: rs itself; for residuals in global memory the
+    // scratch behind the row sums if it holds a block
+    double* asums = reinterpret_cast<double*>(sc);  // min(n, 64 * NR) doubles
+    const bool near = RG && sc_bytes >= 64 * NR * (8 + 16 * gc);
+    z64* part = RG && near ? reinterpret_cast<z64*>(sc + 64 * NR * 8) : rs;
+    const int ldp = near ? 64 * NR : n;
+    for (int r0 = ADJ ? 64 * wave : 0; r0 < n; r0 += ADJ ? 64 * kWaves : 64 * NR) {
+        int i[NR];
+        z64 acc[NR][NG];
+        double asum[NR];
 #pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g)
-            acc[g] = g < gc ? (bg ? ldc<1>(reinterpret_cast<const z64*>(bg) + i + (size_t)g * ldb)
-                                  : ldc<3>(bl + i + (size_t)g * n))
-                            : czero<double>();
-        double asum = 0.0;
-        for (int j0 = 0; j0 < n; j0 += RC) {
-            if (s.real_ops) {
-                const double* __restrict__ Kp = s.K;
-                const double* __restrict__ Mp = s.M;
-                const double* __restrict__ Dp = s.D;
-                double kv[RC], mv[RC], dv[RC];
+        for (int t = 0; t < NR; ++t) {
+            i[t] = min(r0 + lane + 64 * t, n - 1);
+            asum[t] = 0.0;
 #pragma unroll
-                for (int u = 0; u < RC; ++u) {
-                    const int j = min(j0 + u, n - 1);
-                    const int e = ADJ ? j + i * n : i + j * n;
-                    kv[u] = lds1<1>(Kp + e);
-                    mv[u] = lds1<1>(Mp + e);
-                    dv[u] = s.has_D ? lds1<1>(Dp + e) : 0.0;
-                }
-                if (BF) {
-                    // branch-free: columns beyond n contribute zero, and columns
-                    // g >= gc repeat column gc - 1 (their sums are discarded)
-    #pragma unroll
-                    for (int u = 0; u < RC; ++u) {
-                        const bool in = j0 + u < n;
-                        const int j = min(j0 + u, n - 1);
-                        z64 au = cmk<double>(kv[u] - w2 * mv[u], (ADJ ? -1.0 : 1.0) * (s.eta * kv[u] + w * dv[u]));
-                        au.re = in ? au.re : 0.0;
-                        au.im = in ? au.im : 0.0;
-                        if (need_anorm) asum += zabs(au);
-    #pragma unroll
-                        for (int g = 0; g < kMaxGroup; ++g)
-                            cfms(acc[g], au, ldc<3>(xs + j + (size_t)min(g, gc - 1) * n));
+            for (int g = 0; g < NG; ++g) acc[t][g] = czero<double>();
+        }
+        auto column = [&](const z64 (&a)[NR], const z64 (&x)[NG]) {
+            if (need_anorm)
+#pragma unroll
+                for (int t = 0; t < NR; ++t) asum[t] += zabs(a[t]);
+#pragma unroll
+            for (int t = 0; t < NR; ++t)
+#pragma unroll
+                for (int g = 0; g < NG; ++g) cfms(acc[t][g], a[t], x[g]);
+        };
+        auto solution = [&](int j, z64 (&x)[NG]) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) x[g] = ldc<3>(xs + (j + (size_t)min(g, gc - 1) * n));
+        };
+        with_kind(s, [&](auto kc) {
+            constexpr int KIND = decltype(kc)::value;
+            if constexpr (KIND == kOpCplx) {
+#pragma nounroll
+                for (int j = clo; j < chi; ++j) {
+                    z64 a[NR], x[NG];
+                    solution(j, x);
+#pragma unroll
+                    for (int t = 0; t < NR; ++t) {
+                        const z64 e = elem_at<KIND>(s, ADJ ? (size_t)j + (size_t)i[t] * n : (size_t)i[t] + (size_t)j * n, w, w2);
+                        a[t] = ADJ ? cconj(e) : e;
                     }
-                } else {
-    #pragma unroll
+                    column(a, x);
+                }
+            } else {
+                double kv[2][RC][NR], mv[2][RC][NR], dv[2][RC][NR];
+                auto load = [&](int j0, auto bc) {
+                    constexpr int B = decltype(bc)::value;
+#pragma unroll
                     for (int u = 0; u < RC; ++u) {
-                        if (j0 + u < n) {
-                            const z64 au = cmk<double>(kv[u] - w2 * mv[u], (ADJ ? -1.0 : 1.0) * (s.eta * kv[u] + w * dv[u]));
-                            if (need_anorm) asum += zabs(au);
-    #pragma unroll
-                            for (int g = 0; g < kMaxGroup; ++g)
-                                if (g < gc) cfms(acc[g], au, ldc<3>(xs + j0 + u + (size_t)g * n));
+                        const int c = min(j0 + u, n - 1);
+#pragma unroll
+                        for (int t = 0; t < NR; ++t) {
+                            const int e = ADJ ? c + i[t] * n : i[t] + c * n;
+                            kv[B][u][t] = lds1<1>(s.K + e);
+                            mv[B][u][t] = lds1<1>(s.M + e);
+                            dv[B][u][t] = KIND == kOpReal3 ? lds1<1>(s.D + e) : 0.0;
                         }
                     }
+                };
+                auto use = [&](int j0, auto bc) {
+                    constexpr int B = decltype(bc)::value;
+#pragma unroll
+                    for (int u = 0; u < RC; ++u)
+                        if (j0 + u < chi) {
+                            z64 a[NR], x[NG];
+                            solution(j0 + u, x);
+#pragma unroll
+                            for (int t = 0; t < NR; ++t)
+                                a[t] = cmk<double>(kv[B][u][t] - w2 * mv[B][u][t],
+                                                   (ADJ ? -1.0 : 1.0) * (s.eta * kv[B][u][t] + w * dv[B][u][t]));
+                            column(a, x);
+                        }
+                };
+                constexpr std::integral_constant<int, 0> b0{};
+                constexpr std::integral_constant<int, 1> b1{};
+                load(clo, b0);
+#pragma nounroll
+                for (int j0 = clo; j0 < chi; j0 += 2 * RC) {
+                    load(min(j0 + RC, n - 1), b1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    use(j0, b0);
+                    load(min(j0 + 2 * RC, n - 1), b0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    use(j0 + RC, b1);
                 }
-                continue;
             }
-            // complex operators: 4 columns per round
-            for (int j1 = j0; j1 < j0 + RC && j1 < n; j1 += 4) {
-                z64 a[4];
+        });
+        // sums of the shares, one wavefront after the other; the last one adds b
+        for (int q = 0; q < NS; ++q) {
+            if (ADJ || wave == q) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int j = min(j1 + u, n - 1);
-                    a[u] = ADJ ? cconj(assemble_at(s, (size_t)j + (size_t)i * n, w, w2))
-                               : assemble_at(s, (size_t)i + (size_t)j * n, w, w2);
-                }
+                for (int t = 0; t < NR; ++t)
+                    if (r0 + lane + 64 * t < n) {
+                        const int il = near ? lane + 64 * t : i[t];
+                        double as = asum[t];
+                        if (need_anorm) {
+                            if (q > 0) as += asums[lane + 64 * t];
+                            if (q + 1 < NS) asums[lane + 64 * t] = as;
+                            else amax = nmax(amax, as);
+                        }
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (j1 + u < n) {
-                        if (need_anorm) asum += zabs(a[u]);
-#pragma unroll
-                        for (int g = 0; g < kMaxGroup; ++g)
-                            if (g < gc) cfms(acc[g], a[u], ldc<3>(xs + j1 + u + (size_t)g * n));
+                        for (int g = 0; g < NG; ++g)
+                            if (g < gc) {
+                                z64 a = acc[t][g];
+                                if (q > 0) {
+                                    const z64 o = RG ? part[il + (size_t)g * ldp] : ldc<3>(part + il + (size_t)g * ldp);
+                                    a.re += o.re;
+                                    a.im += o.im;
+                                }
+                                if (q + 1 < NS) {
+                                    if (RG) part[il + (size_t)g * ldp] = a;
+                                    else stc<3>(part + il + (size_t)g * ldp, a);
+                                } else {
+                                    const z64 b = bg ? ldc<1>(reinterpret_cast<const z64*>(bg) + i[t] + (size_t)g * ldb)
+                                                     : ldc<3>(bl + i[t] + (size_t)g * n);
+                                    a.re += b.re;
+                                    a.im += b.im;
+                                    if (RG) rs[i[t] + (size_t)g * n] = a;
+                                    else stc<3>(rs + i[t] + (size_t)g * n, a);
+                                }
+                            }
                     }
-                }
             }
+            if (!ADJ) __syncthreads();
         }
-        amax = nmax(amax, asum);
-#pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g)
-            if (g < gc) {
-                if (RG) rs[i + (size_t)g * n] = acc[g];
-                else stc<3>(rs + i + (size_t)g * n, acc[g]);
-            }
     }
-    __syncthreads();
+    if (ADJ) __syncthreads();
+}
+
+template <bool ADJ, bool RG = false>
+__device__ __forceinline__ void residual(const SysDesc& s, double w, double w2, const double2* bg, int ldb,
+                         const z64* bl, const z64* xs, z64* rs, int gc, bool need_anorm,
+                         double* red, char* sc, int sc_bytes, double (&out)[kRedSlots]) {
+    const int n = __builtin_amdgcn_readfirstlane(s.n), tid = threadIdx.x;
+    gc = __builtin_amdgcn_readfirstlane(gc);
+    double amax = 0.0;
+    if (ADJ || gc == 1)
+        residual_rows<ADJ, RG, 1, ADJ ? 8 : 2>(s, w, w2, bg, ldb, bl, xs, rs, 1, need_anorm, sc, sc_bytes, amax);
+    else
+        residual_rows<ADJ, RG, kMaxGroup, 1>(s, w, w2, bg, ldb, bl, xs, rs, gc, need_anorm, sc, sc_bytes, amax);
     // pass 2: the norms of the backward error
     double v[kRedSlots];
 #pragma unroll
@@ -1469,7 +1577,8 @@ __device__ __forceinline__ int solve_group(const SysDesc& s, double w, double w2
     if (!want_berr) return 0;
     for (;;) {
         double out[kRedSlots];
-        residual<ADJ, ResCols<T>::K, BF, RG>(s, w, w2, bg, ldb, bl, xs, rs, gc, *anorm < 0.0, red, out);
+        residual<ADJ, RG>(s, w, w2, bg, ldb, bl, xs, rs, gc, *anorm < 0.0, red,
+                          reinterpret_cast<char*>(wv), n * gc * (int)sizeof(cx<T>), out);
         if (*anorm < 0.0) *anorm = out[0];
         bool conv = true;
 #pragma unroll

@@ -52,21 +52,6 @@ __device__ __forceinline__ double wave_dmax(double v) {
     wave_argmax64(b);
     return __longlong_as_double((long long)b);
 }
-// |a| for the norm of A, scaled by a power of two so that the squares stay in range:
-// an estimate of 1 / sqrt and two Newton steps (1 ulp)
-__device__ __forceinline__ double zabs_fast(z64 a) {
-    const int e = __builtin_amdgcn_frexp_exp(nmax(fabs(a.re), fabs(a.im)));
-    const double x = __builtin_amdgcn_ldexp(a.re, -e), y = __builtin_amdgcn_ldexp(a.im, -e);
-    const double q = fma(x, x, y * y);
-    const double y0 = __builtin_amdgcn_rsq(q);
-    double h = 0.5 * y0, g = q * y0;
-    const double r = fma(-h, g, 0.5);
-    g = fma(g, r, g);
-    h = fma(h, r, h);
-    g = fma(fma(-g, g, q), h, g);
-    return q == 0.0 ? 0.0 : __builtin_amdgcn_ldexp(g, e);
-}
-
 // max |z| over the wavefront's rows (NaN propagates); the squares decide
 // unless they leave the range of a double
 template <int RM>
@@ -78,53 +63,8 @@ __device__ __forceinline__ double wave_zmax(const z64 (&z)[RM]) {
     if ((m > 1e-290 && m < 1e300)) return sqrt(m);
     double h = 0.0;
 #pragma unroll
-    for (int t = 0; t < RM; ++t) h = nmax(h, zabs_fast(z[t]));
+    for (int t = 0; t < RM; ++t) h = nmax(h, zabs(z[t]));
     return wave_dmax(h);
-}
-
-// 1 / z, complex128: z scaled by a power of two to [1, 2) in its larger part,
-// one reciprocal of |z|^2 (hardware estimate and two Newton steps).  Smith's
-// form takes three divisions in a chain; same error (2 ulp against 2.5).
-__device__ __forceinline__ z64 zrecip(z64 z) {
-    const double a = fabs(z.re) >= fabs(z.im) ? z.re : z.im;
-    const int e = -__builtin_amdgcn_frexp_exp(a);
-    const double x = __builtin_amdgcn_ldexp(z.re, e), y = __builtin_amdgcn_ldexp(z.im, e);
-    const double q = fma(x, x, y * y);
-    double r = __builtin_amdgcn_rcp(q);
-    r = fma(fma(-q, r, 1.0), r, r);
-    r = fma(fma(-q, r, 1.0), r, r);
-    return cmk<double>(__builtin_amdgcn_ldexp(x * r, e), __builtin_amdgcn_ldexp(-y * r, e));
-}
-__device__ __forceinline__ cx<float> reg_recip(cx<float> z) { return crecip(z); }
-__device__ __forceinline__ z64 reg_recip(z64 z) { return zrecip(z); }
-
-// ---- operator kinds of the assembly (uniform per point) ------------------------------------------
-enum : int { kOpReal2 = 0, kOpReal3 = 1, kOpCplx = 2 };
-__device__ __forceinline__ int op_kind(const SysDesc& s) {
-    return s.real_ops ? (s.has_D ? kOpReal3 : kOpReal2) : kOpCplx;
-}
-// f(integral_constant<kind>) for the point's kind
-template <typename F>
-__device__ __forceinline__ void with_kind(const SysDesc& s, F&& f) {
-    const int k = op_kind(s);
-    if (k == kOpReal2) f(std::integral_constant<int, kOpReal2>{});
-    else if (k == kOpReal3) f(std::integral_constant<int, kOpReal3>{});
-    else f(std::integral_constant<int, kOpCplx>{});
-}
-// Entry e of A(w), as assemble_at; explicit matrices (op_stride) read the
-// matrix once (M aliases K there).
-template <int KIND>
-__device__ __forceinline__ z64 reg_elem(const SysDesc& s, int e, double w, double w2) {
-    if (KIND == kOpReal2 || KIND == kOpReal3) {
-        const double k = lds1<1>(s.K + e), m = lds1<1>(s.M + e);
-        const double d = KIND == kOpReal3 ? lds1<1>(s.D + e) : 0.0;
-        return cmk<double>(k - w2 * m, s.eta * k + w * d);
-    }
-    const z64 k = ldc<1>(reinterpret_cast<const z64*>(s.K) + e);
-    z64 m = k, d = czero<double>();
-    if (!s.op_stride) m = ldc<1>(reinterpret_cast<const z64*>(s.M) + e);
-    if (s.has_D) d = ldc<1>(reinterpret_cast<const z64*>(s.D) + e);
-    return cmk<double>(k.re - s.eta * k.im - w2 * m.re - w * d.im, k.im + s.eta * k.re - w2 * m.im + w * d.re);
 }
 
 // ---- pivot search of one column (its wavefront) ----------------------------------------------------
@@ -182,7 +122,7 @@ __device__ __forceinline__ void reg_pivot(const cx<T> (&col)[RM], const int (&lp
 // Fast form of the search: the high words of |re| + |im| alone (complex64: the whole
 // word).  True when one row has the largest and its magnitude is far from both
 // ends of the range, so that neither ties, zeros, infinities and NaN nor a
-// scaled reciprocal have to be thought of (reg_pivot and reg_recip do that).
+// scaled reciprocal have to be thought of (reg_pivot and crecip do that).
 template <typename T, int RM>
 __device__ __forceinline__ bool reg_pivot_fast(const cx<T> (&col)[RM], const int (&lpos)[RM], int jj, int& pw) {
     unsigned hi[RM], m = 0;
@@ -311,7 +251,7 @@ __device__ __forceinline__ int reg_eliminate(cx<T> (&x)[CPW][RM], cx<T> (&b)[NE 
                 pw = pln | (tw << 6);
                 const cx<T> pv = pivot_entry(x[j], pw);
                 const bool zero = pv.re == T(0) && pv.im == T(0);
-                rp = reg_recip(pv);
+                rp = crecip(pv);
                 rp.re = zero ? T(0) : rp.re;
                 rp.im = zero ? T(0) : rp.im;
                 if (zero && lane == 0 && lds1<3>(R.sc + 12) == 0) stc1i(R.sc + 12, jj + 1);
@@ -572,7 +512,7 @@ __device__ __forceinline__ void reg_point_refined(const SysDesc* sp, int fidx, c
                     for (int q = 0; q < QC; ++q)
 #pragma unroll
                         for (int t = 0; t < RM; ++t)
-                            a[q][t] = reg_elem<KIND>(s, row[t] + min(reg_col<NW, CPW>(qc + q, 0, wave), n - 1) * n, w, w2);
+                            a[q][t] = elem_at<KIND>(s, row[t] + min(reg_col<NW, CPW>(qc + q, 0, wave), n - 1) * n, w, w2);
                 } else {
 #pragma unroll
                     for (int q = 0; q < QC; ++q)
@@ -586,7 +526,7 @@ __device__ __forceinline__ void reg_point_refined(const SysDesc* sp, int fidx, c
                         const bool ok = in[t] && reg_col<NW, CPW>(qc + q, 0, wave) < n;
                         a[q][t].re = ok ? a[q][t].re : 0.0;
                         a[q][t].im = ok ? a[q][t].im : 0.0;
-                        if (any) asum[t] += zabs_fast(a[q][t]);
+                        if (any) asum[t] += zabs(a[q][t]);
                         x[qc + q][t] = to_t<float>(a[q][t]);
                     }
                 __builtin_amdgcn_sched_barrier(0);  // one chunk's operator loads in flight at a time
@@ -720,7 +660,7 @@ __device__ __forceinline__ void reg_point_refined(const SysDesc* sp, int fidx, c
                     for (int q = 0; q < QC; ++q)
 #pragma unroll
                         for (int t = 0; t < RM; ++t)
-                            a[q][t] = reg_elem<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
+                            a[q][t] = elem_at<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
 #pragma unroll
                     for (int q = 0; q < QC; ++q) {
                         const int c = c0 + q;
@@ -889,7 +829,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
                         for (int q = qc; q < qc + 4; ++q)
 #pragma unroll
                             for (int t = 0; t < RM; ++t)
-                                x[q][t] = reg_elem<KIND>(s, row[t] + min(reg_col<NW, CPW>(q, 0, wave), n - 1) * n, w, w2);
+                                x[q][t] = elem_at<KIND>(s, row[t] + min(reg_col<NW, CPW>(q, 0, wave), n - 1) * n, w, w2);
                     } else {
 #pragma unroll
                         for (int q = qc; q < qc + 4; ++q)
@@ -987,14 +927,14 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
                             for (int q = 0; q < 4; ++q)
 #pragma unroll
                                 for (int t = 0; t < RM; ++t)
-                                    a[q][t] = reg_elem<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
+                                    a[q][t] = elem_at<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
 #pragma unroll
                             for (int q = 0; q < 4; ++q)
                                 if (c0 + q < n) {
                                     const z64 xc = ldc<3>(vw + c0 + q);
 #pragma unroll
                                     for (int t = 0; t < RM; ++t) {
-                                        as[t] += zabs_fast(a[q][t]);
+                                        as[t] += zabs(a[q][t]);
                                         cfms(r[t], a[q][t], xc);
                                     }
                                 }
