@@ -1132,11 +1132,7 @@ __device__ __forceinline__ void lower_h_unit_solve(const TriCtx<T>& t, cx<T>* w,
 // rows outside the block from its prefetched 16 entries (further rows of
 // n > 256 load theirs on demand).  FWD: blocks in increasing order (lower
 // triangular op), else decreasing.  TRANS: op(LU)(i, k) = conj(LU(k, i)).
-// BF: the inverse-apply and off-diagonal loops without branches (entries
-// beyond the block contribute zero, right-hand sides g >= gc repeat column
-// gc - 1 and are discarded, all 16 entries of a row are loaded); more
-// registers, used by the complex64 wide-panel kernel only.
-template <typename T, bool FWD, bool INV, bool UNIT, bool TRANS, bool BF = false>
+template <typename T, bool FWD, bool INV, bool UNIT, bool TRANS>
 __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* __restrict__ binv, cx<T>* w,
                                                int gc) {
     constexpr int B = 16;
@@ -1168,7 +1164,7 @@ __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* 
         for (int u = 0; u < B; ++u) {
             // rows outside the update are loaded (clamped) but never used; entries
             // beyond kb (narrow blocks of the register-panel kernel) are not loaded
-            if (BF || u < kb) {
+            if (u < kb) {
                 const int k = k0 + min(u, kb - 1);
                 r[u] = TRANS ? ldc<1>(LU + ((size_t)lds1<3>(t.rmap + k) + (size_t)i0c * ld))
                              : ldc<1>(LU + (pr0 + (size_t)k * ld));
@@ -1199,14 +1195,7 @@ __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* 
                 cx<T> acc = czero<T>();
 #pragma unroll
                 for (int k = 0; k < B; ++k) {
-                    if (BF) {
-                        cx<T> d = ldc<3>(Dg + (r + k * B));
-                        d.re = k < kb ? d.re : T(0);
-                        d.im = k < kb ? d.im : T(0);
-                        cfma(acc, d, ldc<3>(y + min(k, kb - 1)));
-                    } else if (k < kb) {
-                        cfma(acc, ldc<3>(Dg + (r + k * B)), ldc<3>(y + k));
-                    }
+                    if (k < kb) cfma(acc, ldc<3>(Dg + (r + k * B)), ldc<3>(y + k));
                 }
                 if (r < kb) stc<3>(y + r, acc);  // one wave: every read above precedes the writes
             }
@@ -1249,15 +1238,7 @@ __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* 
             for (int g = 0; g < kMaxGroup; ++g) acc[g] = czero<T>();
 #pragma unroll
             for (int u = 0; u < B; ++u) {
-                if (BF) {
-                    cx<T> a = CONJ ? cconj(rc[u]) : rc[u];
-                    a.re = u < kb ? a.re : T(0);
-                    a.im = u < kb ? a.im : T(0);
-                    const int uc = min(u, kb - 1);
-#pragma unroll
-                    for (int g = 0; g < kMaxGroup; ++g)
-                        cfma(acc[g], a, ldc<3>(w + (k0 + uc + (size_t)min(g, gc - 1) * n)));
-                } else if (u < kb) {
+                if (u < kb) {
                     const cx<T> a = CONJ ? cconj(rc[u]) : rc[u];
 #pragma unroll
                     for (int g = 0; g < kMaxGroup; ++g)
@@ -1278,6 +1259,146 @@ __device__ __forceinline__ void tri_solve_pipe(const TriCtx<T>& t, const cx<T>* 
         dc = dn;
 #pragma unroll
         for (int u = 0; u < B; ++u) rc[u] = rn[u];
+    }
+    __syncthreads();
+}
+
+// ---- the same solves of complex64 factors on the matrix cores ------------------------------
+// L y = w (FWD, unit diagonal) or U y = w for up to four right-hand sides, 16-row blocks with
+// stored inverses (binv).  Row tile t = kWaves * (4 rg + q) + wave belongs to lanes 16 q .. 16 q + 15 of
+// its wavefront, one row a lane, and stays in accumulators of 4x4x1 products: the four
+// right-hand sides are the A operand (a block's 16 solved rows are one register, row k
+// selected by broadcasting its block of four lanes) and 64 rows of L the B operand, as they
+// come from the slot.  Per block: the owner of its tile applies the inverse (16x16x4
+// products: columns re and im of the right-hand sides) and publishes y in LDS; after one barrier
+// every wavefront subtracts the block's columns from its rows, with the next block's
+// columns in flight.
+//
+// Bound by that chain and by the slot's way from the caches.  The form above (one row a
+// thread, solved rows read entry by entry from LDS, two barriers per block) took 5.4k cycles per
+// 16-row block at n = 256 with the GPU otherwise idle, this one 2.6k
+// (n = 1024: 16.6k and 8.8k with every CU busy)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+typedef float tri_f4 __attribute__((ext_vector_type(4)));
+
+template <int NRG, bool FWD>
+__device__ __forceinline__ void tri_solve_mfma(const TriCtx<float>& t, const cx<float>* __restrict__ binv, cx<float>* w,
+                                               int gc) {
+    constexpr int B = 16, ZL = 20;  // ZL: leading dimension of a block in LDS
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = __builtin_amdgcn_readfirstlane(t.n), ld = __builtin_amdgcn_readfirstlane(t.ld);
+    gc = __builtin_amdgcn_readfirstlane(gc);
+    const int nb = (n + B - 1) / B;
+    const cx<float>* __restrict__ LU = t.LU;
+    auto stf = [](float* p, float v) { *(__attribute__((address_space(3))) float*)p = v; };
+    float* zb = reinterpret_cast<float*>(t.Dg);  // the owner's block [8 columns][ZL]: re of 4, im of 4
+    float* yb = zb + 8 * ZL;                     // solved blocks, two buffers of [re, im][16 rows][4]
+    int row[NRG];
+    int pr[NRG];
+    tri_f4 re[NRG], im[NRG];
+#pragma unroll
+    for (int rg = 0; rg < NRG; ++rg) {
+        row[rg] = B * (kWaves * (4 * rg + lg) + wave) + li;
+        const int rc = min(row[rg], n - 1);
+        pr[rg] = lds1<3>(t.rmap + rc);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const cx<float> v = ldc<3>(w + (rc + (size_t)min(g, gc - 1) * n));
+            const bool ok = row[rg] < n && g < gc;
+            re[rg][g] = ok ? v.re : 0.f;
+            im[rg][g] = ok ? v.im : 0.f;
+        }
+    }
+    // columns k0 .. k0+15 of this lane's rows that are still to be solved
+    auto load_cols = [&](int b, cx<float> (&l)[NRG][B]) {
+        const int k0 = b * B, kl = min(B, n - k0) - 1;
+#pragma unroll
+        for (int rg = 0; rg < NRG; ++rg)
+            if (FWD ? row[rg] >= k0 + B : row[rg] < k0)
+#pragma unroll
+                for (int k = 0; k < B; ++k) l[rg][k] = ldc<1>(LU + (pr[rg] + (size_t)(k0 + min(k, kl)) * ld));
+    };
+    // operands of the inverse of block b: row li, columns 4 lg + s
+    auto load_inv = [&](int b, cx<float> (&a)[4]) {
+        const int kb = min(B, n - b * B);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            a[s] = ldc<1>(binv + ((size_t)b * B * B + min(li, kb - 1) + min(4 * lg + s, kb - 1) * kb));
+    };
+    cx<float> l0[NRG][B], l1[NRG][B], inv[4];
+    auto step = [&](int st, const cx<float> (&lc)[NRG][B], cx<float> (&lnext)[NRG][B]) {
+        const int b = FWD ? st : nb - 1 - st, k0 = b * B, kb = min(B, n - k0);
+        float* yc = yb + (st & 1) * 8 * B;
+        if (st + 1 < nb) load_cols(FWD ? b + 1 : b - 1, lnext);
+        if (wave == b % kWaves) {
+            const int tq = b / kWaves;
+#pragma unroll
+            for (int rg = 0; rg < NRG; ++rg)
+                if (tq / 4 == rg && lg == (tq & 3)) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {  // rows beyond kb are zero: their lanes hold rows >= n
+                        stf(zb + g * ZL + li, row[rg] < n ? re[rg][g] : 0.f);
+                        stf(zb + (4 + g) * ZL + li, row[rg] < n ? im[rg][g] : 0.f);
+                    }
+                }
+            __builtin_amdgcn_wave_barrier();
+            const int c8 = li & 7;
+            const tri_f4 z1 = *(const __attribute__((address_space(3))) tri_f4*)(zb + c8 * ZL + 4 * lg);
+            const tri_f4 z2 = *(const __attribute__((address_space(3))) tri_f4*)(zb + (c8 ^ 4) * ZL + 4 * lg);
+            tri_f4 y1 = {0.f, 0.f, 0.f, 0.f}, y2 = y1;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[s].re, z1[s], y1, 0, 0, 0);
+                y2 = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[s].im, c8 < 4 ? -z2[s] : z2[s], y2, 0, 0, 0);
+            }
+            const int bo = FWD ? b + kWaves : b - kWaves;  // the next block of this wavefront
+            if (li < 8) {
+                const int g = li & 3, part = li >> 2;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int k = 4 * lg + r;
+                    const float y = k < kb ? y1[r] + y2[r] : 0.f;
+                    stf(yc + part * 4 * B + k * 4 + g, y);
+                    if (k < kb && g < gc) stf(reinterpret_cast<float*>(w + (k0 + k + (size_t)g * n)) + part, y);
+                }
+            }
+            if (bo >= 0 && bo < nb) load_inv(bo, inv);
+        }
+        __syncthreads();
+        const float yr = lds1<3>(yc + lane), yi = lds1<3>(yc + 4 * B + lane);
+        const float nr = -yr, ni = -yi;
+#pragma unroll
+        for (int rg = 0; rg < NRG; ++rg) {
+            // a row of this group is left: its last (FWD) or first tile
+            const int tl = kWaves * (4 * rg + (FWD ? 3 : 0)) + wave;
+            if (FWD ? tl > b : tl < b)
+                static_for_seq([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    re[rg] = __builtin_amdgcn_mfma_f32_4x4x1f32(nr, lc[rg][k].re, re[rg], 4, k, 0);
+                    im[rg] = __builtin_amdgcn_mfma_f32_4x4x1f32(nr, lc[rg][k].im, im[rg], 4, k, 0);
+                    re[rg] = __builtin_amdgcn_mfma_f32_4x4x1f32(yi, lc[rg][k].im, re[rg], 4, k, 0);
+                    im[rg] = __builtin_amdgcn_mfma_f32_4x4x1f32(ni, lc[rg][k].re, im[rg], 4, k, 0);
+                }, std::make_integer_sequence<int, B>{});
+        }
+    };
+#pragma unroll
+    for (int rg = 0; rg < NRG; ++rg)
+#pragma unroll
+        for (int k = 0; k < B; ++k) l0[rg][k] = l1[rg][k] = czero<float>();
+    load_cols(FWD ? 0 : nb - 1, l0);
+    {
+        // the first block of this wavefront in the order of the solve
+        const int b0 = FWD ? wave : nb - 1 - ((nb - 1 - wave) % kWaves + kWaves) % kWaves;
+        if (b0 >= 0 && b0 < nb) load_inv(b0, inv);
+    }
+#pragma nounroll
+    for (int st = 0; st < nb; st += 2) {
+        step(st, l0, l1);
+        if (st + 1 < nb) step(st + 1, l1, l0);
     }
     __syncthreads();
 }
@@ -1534,7 +1655,7 @@ __device__ __forceinline__ double backward_error(double rmax, double anorm, doub
 // On entry wv holds P b (permuted, type T) for gc columns and xs/rs are free.
 // On exit xs holds the solution (FP64).  Returns refinement steps; conv[] = 1
 // for columns meeting tol; berr_out[] their backward errors (when computed).
-template <typename T, bool ADJ, bool BF = false, bool RG = false>
+template <typename T, bool ADJ, int NRG = 0, bool RG = false>
 __device__ __forceinline__ int solve_group(const SysDesc& s, double w, double w2, const TriCtx<T>& tri,
                            const int* perm, cx<T>* wv, z64* xs, z64* rs, int gc,
                            const double2* bg, int ldb, const z64* bl, bool refine, bool want_berr,
@@ -1546,10 +1667,14 @@ __device__ __forceinline__ int solve_group(const SysDesc& s, double w, double w2
     // so the first solve is the U solve only
     auto solve_t = [&]() {
         if (tri.rmap) {  // factors in the global slot: pipelined block solves
-            if (!ADJ) {
+            if constexpr (NRG > 0) {
                 if (fwd_done) fwd_done = false;
-                else tri_solve_pipe<T, true, true, true, false, BF>(tri, tri.Linv, wv, gc);
-                if (tri.inv_u) tri_solve_pipe<T, false, true, false, false, BF>(tri, tri.Uinv, wv, gc);
+                else tri_solve_mfma<NRG, true>(tri, tri.Linv, wv, gc);
+                tri_solve_mfma<NRG, false>(tri, tri.Uinv, wv, gc);
+            } else if (!ADJ) {
+                if (fwd_done) fwd_done = false;
+                else tri_solve_pipe<T, true, true, true, false>(tri, tri.Linv, wv, gc);
+                if (tri.inv_u) tri_solve_pipe<T, false, true, false, false>(tri, tri.Uinv, wv, gc);
                 else tri_solve_pipe<T, false, false, false, false>(tri, nullptr, wv, gc);
             } else {
                 tri_solve_pipe<T, true, false, false, true>(tri, nullptr, wv, gc);
@@ -1926,18 +2051,17 @@ __device__ __forceinline__ void process_point(const SysDesc& s, int fidx, const 
         __syncthreads();
         double be[kMaxGroup];
         bool conv;
-        // branch-free residual rounds in the complex64 wide-panel kernel (the
-        // others spill with them); residuals in LDS, or in the slot (a copy of
-        // the loop with generic accesses to them)
+        // complex64 wide panels: triangular solves on the matrix cores
         constexpr bool BF = WIDE != 0 && sizeof(T) == 4;
+        constexpr int NRG = !BF ? 0 : MAXR > kWaves ? MAXR / kWaves : 1;
         if (BF) __builtin_amdgcn_s_setprio(2);
         int it;
         if (kRsg && rsg)
-            it = solve_group<T, false, BF, kRsg>(s, w, w2, tri, L.rmap, wv, xs, rs_slot, gc, Fg, s.ldf,
+            it = solve_group<T, false, NRG, kRsg>(s, w, w2, tri, L.rmap, wv, xs, rs_slot, gc, Fg, s.ldf,
                                                  nullptr, refine, want_berr, kp.tol, kp.max_iter,
                                                  &anorm, be, &conv, L.red, fwd);
         else
-            it = solve_group<T, false, BF, false>(s, w, w2, tri, L.rmap, wv, xs, rs, gc, Fg, s.ldf,
+            it = solve_group<T, false, NRG, false>(s, w, w2, tri, L.rmap, wv, xs, rs, gc, Fg, s.ldf,
                                                   nullptr, refine, want_berr, kp.tol, kp.max_iter,
                                                   &anorm, be, &conv, L.red, fwd);
         if (BF) __builtin_amdgcn_s_setprio(0);
