@@ -5,8 +5,8 @@ by a blocked factorisation; either can also run as
   - the 16-column register panel (kernel 1: three workgroups per CU for
     complex64, two for complex128), or
   - the wide LDS panel (kernel 2) with 160 KiB of LDS per workgroup (one per
-    CU, panels up to 64 columns) or 80 KiB (two per CU, up to 32), with the
-    panel width capped or not,
+    CU, eight wavefronts above n = 512, complex128 256) or 80 KiB (two per CU), panels
+    of up to 32 columns (complex128 16), with the width capped or not,
 and which is fastest depends on the order n, the right-hand sides and the
 mode.  tune() times every candidate on a sample of the caller's frequencies
 (inputs and outputs resident on the device, HIP events on the launch stream),
@@ -34,12 +34,8 @@ CANDIDATES = [
     ("wide-2perCU", 2, 80 * 1024, 0),
     ("wide-2perCU-jb16", 2, 80 * 1024, 16),
     ("wide-1perCU", 2, 160 * 1024 - 256, 0),
-    ("wide-1perCU-jb32", 2, 160 * 1024 - 256, 32),
-    # two-level update: several LDS panels per 64-column step (32 complex128),
-    # one deferred update of the columns right of the step
-    ("wide-2level-2perCU", 4, 80 * 1024, 0),
-    ("wide-2level-1perCU", 4, 160 * 1024 - 256, 0),
-    # Gauss 3M complex products in the trailing update (complex64 only)
+    # Gauss 3M complex products in the update of the panels (complex64 only; above
+    # n = 256 the same as kernel 2)
     ("wide-3M-2perCU", 3, 80 * 1024, 0),
     ("wide-3M-1perCU", 3, 160 * 1024 - 256, 0),
     # the library's own choice (up to n = 128: systems in registers)
@@ -97,9 +93,7 @@ def automatic_name(n, mode):
     if n <= 128:
         return "automatic"
     one_per_cu = n > (512 if complex64 else 256)
-    if n > 256:  # the two-level update (complex128 beyond n = 512: register panel either way)
-        return "wide-2level-1perCU" if one_per_cu else "wide-2level-2perCU"
-    if complex64:  # Gauss 3M products up to n = 256
+    if complex64 and n <= 256:  # Gauss 3M products
         return "wide-3M-2perCU"
     return "wide-1perCU" if one_per_cu else "wide-2perCU"
 

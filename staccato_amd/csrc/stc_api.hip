@@ -86,10 +86,9 @@ struct LaunchOrder {
 
 // How the blocked path of a launch runs (stc_policy): kernel 0 = automatic,
 // 1 = 16-column register panel, 2 = wide LDS panel, 3 = wide LDS panel with
-// Gauss 3M products in the trailing update (complex64; else as 2), 4 = wide LDS
-// panel with the two-level update (several LDS panels per step, one deferred
-// rank-64 / rank-32 update of the columns right of the step); lds_budget bytes per
-// workgroup (0 = automatic); jb_max caps the panel width (0 = none).
+// Gauss 3M products in the update of the panels (complex64 up to n = 256; else as 2),
+// 4 = as 2; lds_budget bytes per workgroup (0 = automatic); jb_max caps the panel
+// width (0 = none).
 struct Policy {
     int kernel = 0;
     int lds_budget = 0;
@@ -220,8 +219,7 @@ int plan_systems(SysDesc* sys, int nsys, int ts, int adj, int jb_cap, int maxr, 
 
 // Wide-panel layout of every system within `budget` bytes of LDS; false when
 // one of them does not fit.
-bool layout_wide(SysDesc* sys, int nsys, int ts, int adj, int jb_cap, int maxr, int budget,
-                 bool two_level, int* lds_out) {
+bool layout_wide(SysDesc* sys, int nsys, int ts, int adj, int jb_cap, int maxr, int budget, int* lds_out) {
     int lds = 0;
     for (int i = 0; i < nsys; ++i) {
         const Layout L = plan_layout_wide(sys[i].n, sys[i].nrhs, ts, budget, jb_cap, adj, maxr);
@@ -235,10 +233,6 @@ bool layout_wide(SysDesc* sys, int nsys, int ts, int adj, int jb_cap, int maxr, 
         sys[i].lay_cw = L.cw;
         sys[i].lay_G = L.G;
         sys[i].lay_rsg = L.rsg;
-        // two-level update: steps of the widest panel the trailing update holds
-        // (64 columns complex64, 32 complex128), a multiple of the LDS panel
-        const int jmax = wide_jb_max(ts);
-        sys[i].lay_jo = (two_level && !L.small && L.jb >= kSB && L.jb < jmax) ? (jmax / L.jb) * L.jb : 0;
     }
     *lds_out = lds;
     return true;
@@ -263,7 +257,7 @@ Policy policy_for(const stc_ctx* h, int n, int refine) {
 struct LaunchCfg {
     int refine = 0;
     int maxr = 1;
-    int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path, 2 with 3M products, 3 two-level;
+    int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path, 2 with 3M products;
                     // reg_kernel: 4, with the adjoint 5
     int threads = kThreads;
     int lds = 0;
@@ -338,20 +332,13 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
     // automatic: systems that need a factor slot go to the wide-panel kernel
     // when the largest order exceeds 128 (below, the register panel at three
     // workgroups per CU measured faster), the kernel is built for these rows
-    // per lane and every system's panel fits its LDS; policy kernels 2 and 3
-    // take it for every launch it fits (3: Gauss 3M products, complex64 only)
+    // per lane and every system's panel fits its LDS; policy kernels 2, 3 and 4
+    // take it for every launch it fits
     bool blocked = false;
     for (int i = 0; i < nsys; ++i) blocked = blocked || !sys[i].lay_small;
     cfg->wide = 0;
-    // automatic: the two-level update above n = 256 (measured on MI355X, both
-    // modes: n = 384 +11 % / +7 %, 512 +24 % / +12 %, 1024 +36 % complex64),
-    // one level up to n = 256 (there two-level loses for complex64: 374k
-    // against 457k points/s at n = 256), with Gauss 3M products for complex64
-    // (n = 160 / 192 / 224 / 256: +1.5 / +5.3 / +4.8 / +3.5 % over 4M)
-    const bool two_auto = pol.kernel == 0 && maxn > 256;
-    const bool g3_auto = pol.kernel == 0 && refine && maxn <= 256;
-    const int wkind = ((pol.kernel == 3 || g3_auto) && sweep_kernel_fn(refine, maxr, 2)) ? 2
-                      : ((pol.kernel == 4 || two_auto) && sweep_kernel_fn(refine, maxr, 3)) ? 3 : 1;
+    // automatic: Gauss 3M products for complex64 up to n = 256 (built only there)
+    const int wkind = (pol.kernel == 3 || pol.kernel == 0) && sweep_kernel_fn(refine, maxr, 2) ? 2 : 1;
     if (((pol.kernel == 0 && blocked && maxn > 128) || pol.kernel >= 2) && sweep_kernel_fn(refine, maxr, wkind)) {
         int wcap = wide_jb_max(ts);
         if (pol.jb_max > 0) wcap = std::max(kSB, std::min(pol.jb_max, wcap));
@@ -361,7 +348,7 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
         const int auto_budget = maxn > (ts == 8 ? 512 : 256) ? kBudgetLarge : kBudgetSmall;
         const int budget = pol.lds_budget > 0 ? pol.lds_budget : auto_budget;
         int lds = 0;
-        if (layout_wide(sys, nsys, ts, adj, wcap, maxr, budget, wkind == 3, &lds)) {  // writes only when all fit
+        if (layout_wide(sys, nsys, ts, adj, wcap, maxr, budget, &lds)) {  // writes only when all fit
             cfg->wide = wkind;
             cfg->lds = lds;
         }

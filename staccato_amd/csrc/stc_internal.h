@@ -19,7 +19,7 @@ namespace stc {
 // was exposed (512 points: n = 1024 refined, 16 right-hand sides 108.4 -> 64.4 ms;
 // n = 512 plain, 4 right-hand sides 12.3 -> 11.0 ms).
 __host__ __device__ constexpr int sweep_threads(int refine, int maxr, int wide) {
-    return wide >= 1 && wide <= 3 && maxr >= (refine ? 16 : 8) ? 512 : 256;
+    return wide >= 1 && wide <= 2 && maxr >= (refine ? 16 : 8) ? 512 : 256;
 }
 #ifdef STC_INST_WIDE
 constexpr int kThreads = sweep_threads(STC_INST_REFINE, STC_INST_MAXR, STC_INST_WIDE);
@@ -85,7 +85,6 @@ struct SysDesc {
     int lay_jb;
     int lay_cw;
     int lay_G;
-    int lay_jo;          // wide path: outer width of the two-level update (<= lay_jb: none)
     int lay_rsg;         // wide path: FP64 residuals in the factor slot instead of LDS
 };
 
@@ -111,7 +110,6 @@ struct Layout {
     int cw;         // trailing column chunk width (blocked)
     int G;          // right-hand sides per solve group
     int lds;        // bytes needed
-    int jo = 0;     // wide path: columns per two-level step (<= jb: one level)
     int rsg = 0;    // wide path: FP64 residuals in the factor slot (frees LDS for the group)
 };
 
@@ -211,9 +209,9 @@ inline Layout plan_layout(int n, int nrhs, int ts, int budget, int jb_cap, int a
 // ---- wide-panel blocked path (sweep_kernel<T, MAXR, true>) ----------------------------
 constexpr int kSB = 16;  // sub-panel width and inverted diagonal block size
 
-// Widest panel the wide kernel keeps in registers for the trailing update:
-// 64 columns for complex64, 32 for complex128.
-__host__ __device__ constexpr int wide_jb_max(int elem_bytes) { return elem_bytes == 8 ? 64 : 32; }
+// Widest panel of the wide kernel: the columns its accumulators hold in the
+// left-looking update, 32 for complex64, 16 for complex128.
+__host__ __device__ constexpr int wide_jb_max(int elem_bytes) { return elem_bytes == 8 ? 32 : 16; }
 
 // LDS of the wide path beyond lds_fixed_bytes: the n x jb panel (leading
 // dimension rounded up to odd, so its columns start in different banks), its inverted

@@ -31,21 +31,6 @@
 namespace stc {
 
 // ---- wavefront maxima ------------------------------------------------------------------------
-template <int CTRL, int RM>
-__device__ __forceinline__ unsigned umax_step(unsigned v) {
-    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xF, false);
-    return o > v ? o : v;
-}
-// maximum over the wavefront, uniform
-__device__ __forceinline__ unsigned wave_umax(unsigned v) {
-    v = umax_step<kDppXor1, 0xF>(v);
-    v = umax_step<kDppXor2, 0xF>(v);
-    v = umax_step<kDppHalfMirror, 0xF>(v);
-    v = umax_step<kDppMirror, 0xF>(v);
-    v = umax_step<kDppRowBcast15, 0xA>(v);
-    v = umax_step<kDppRowBcast31, 0xC>(v);
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
 // maximum of non-negative doubles (NaN counts as the largest, so it propagates)
 __device__ __forceinline__ double wave_dmax(double v) {
     unsigned long long b = (unsigned long long)__double_as_longlong(v) & 0x7FFFFFFFFFFFFFFFull;

@@ -1,25 +1,19 @@
 // stc_wide.h -- wide-panel blocked LU of the sweep kernel (gfx950).
 //
-// The blocked path of sweep_kernel<T, MAXR, 1> (<T, MAXR, 2>: Gauss 3M
-// products in the trailing update; <T, MAXR, 3>: two-level update).  It factors A(w) in the workgroup's
-// global factor slot, right-looking, with panels of jb = 16..64 columns held
-// in LDS (one or two workgroups per CU), and cuts the trailing-matrix traffic
-// by jb / 16 against a 16-column panel:
+// The blocked path of sweep_kernel<T, MAXR, 1> (<T, MAXR, 2>: Gauss 3M products in the
+// panels' update).  It factors A(w) in the workgroup's global factor slot, left-looking,
+// in steps of 32 columns (complex64) or 16 (complex128), with panels of jb columns (a
+// step, or half a complex64 one) held in LDS, one or two workgroups per CU:
 //
-//   panel (m = n - j0 rows x jb columns, LDS, logical row order, assembled
-//   from the operators at j0 = 0):
+//   step: its columns, assembled from the operators, are brought up to date with all
+//   finished columns in the MFMA accumulators of the workgroup (left_update) and
+//   go to the LDS panel (m rows x jb columns, logical row order):
 //     per 16-column sub-panel: pivoted LU with the rows distributed over the
-//     threads (thread t holds rows t + 256 u in registers, one barrier per
+//     threads (a thread's rows in registers, one barrier per
 //     column), rows permuted in the LDS panel afterwards; the 16 x 16
 //     unit-lower diagonal block inverted (one entry per thread); the panel's
 //     remaining columns updated on MFMA (U rows = Linv A, rows below -= L21 U);
-//   trailing columns (matrix, then the first right-hand sides), 16 per chunk,
-//     one wavefront per chunk, no block barrier:
-//     U12 = L11^{-1} A12 by block forward substitution on MFMA in registers
-//     (16-row blocks: acc_b -= L_ba U_a, U_b = Linv_b acc_b), U12 to the slot,
-//     then C -= L21 U12 over tiles of 16 TA rows, the next tile's C loaded
-//     before the current tile's products (assembled from the operators at the
-//     first panel).
+//   the first right-hand sides are the last step's columns, without a panel.
 //
 // Rows never move in the slot (row map, as in the 16-column path); only the
 // LDS panel is kept in logical order.  Complex products take four real MFMAs
@@ -33,15 +27,6 @@
 #pragma once
 
 namespace stc {
-
-// Largest number of 16-row blocks of a wide panel kept in registers.
-constexpr int kPB = 8;  // panel columns loaded per batch
-
-template <typename T>
-struct WideCfg {
-    static constexpr int NB = wide_jb_max(2 * sizeof(T)) / kSB;  // jb <= 64 (complex64), 32 (complex128)
-    static constexpr int TA = sizeof(T) == 4 ? 4 : 2;  // 16-row MFMA tiles per C tile
-};
 
 // d += a * b (complex; a from the lane's A operand, b its B operand).
 template <typename T>
@@ -135,8 +120,51 @@ __device__ __forceinline__ void wave_argmax64(unsigned long long& v) {
     const unsigned l = (unsigned)__builtin_amdgcn_readlane((int)v, 63);
     v = ((unsigned long long)h << 32) | l;
 }
+// maximum over the wavefront of one word, uniform
+template <int CTRL, int RM>
+__device__ __forceinline__ unsigned umax_step(unsigned v) {
+    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xF, false);
+    return o > v ? o : v;
+}
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+    v = umax_step<kDppXor1, 0xF>(v);
+    v = umax_step<kDppXor2, 0xF>(v);
+    v = umax_step<kDppHalfMirror, 0xF>(v);
+    v = umax_step<kDppMirror, 0xF>(v);
+    v = umax_step<kDppRowBcast15, 0xA>(v);
+    v = umax_step<kDppRowBcast31, 0xC>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
 __device__ __forceinline__ void stc1i(int* p, int v) { *(__attribute__((address_space(3))) int*)(p) = v; }
 __device__ __forceinline__ void stc1u(unsigned* p, unsigned v) { *(__attribute__((address_space(3))) unsigned*)(p) = v; }
+
+// This wavefront's candidate, uniform: (hk, lo) of the largest, packed in one word for
+// complex64 (hk < 2^32).  complex128: one 32-bit maximum of the keys' high words and a
+// ballot, the full lexicographic reduction (three words a step) only where rows
+// tie there (n = 256 plain 10.9 -> 10.3 ms); complex64 measured 2 % slower so.
+template <typename T>
+__device__ __forceinline__ unsigned long long wave_candidate(unsigned long long& hk, unsigned& lo) {
+    if constexpr (sizeof(T) == 4) {
+        unsigned long long pk = (hk << 20) | lo;
+        wave_argmax64(pk);
+        hk = pk >> 20;
+        lo = (unsigned)(pk & 0xFFFFFull);
+        return pk;
+    } else {
+        const unsigned h = hk ? (unsigned)(hk >> 32) + 1u : 0u;
+        const unsigned long long b = __ballot(h == wave_umax(h));
+        if ((b & (b - 1)) == 0) {
+            const int src = __builtin_ctzll(b);
+            const unsigned kh = (unsigned)__builtin_amdgcn_readlane((int)(hk >> 32), src);
+            const unsigned kl = (unsigned)__builtin_amdgcn_readlane((int)hk, src);
+            hk = ((unsigned long long)kh << 32) | kl;
+            lo = (unsigned)__builtin_amdgcn_readlane((int)lo, src);
+        } else {
+            wave_argmax_packed(hk, lo);
+        }
+        return 0;
+    }
+}
 
 // Rows moved by a sub-panel's pivoting (the list mvl, sc[12] entries): their
 // entries in the other panel columns and in the row map follow; every source
@@ -244,15 +272,7 @@ __device__ __forceinline__ void subpanel_factor(cx<T>* __restrict__ P, int m, in
                 hk = better ? k : hk;
                 lo = better ? l : lo;
             }
-            unsigned long long pk = 0;
-            if (sizeof(T) == 4) {
-                pk = (hk << 20) | lo;
-                wave_argmax64(pk);
-                hk = pk >> 20;
-                lo = (unsigned)(pk & 0xFFFFFull);
-            } else {
-                wave_argmax_packed(hk, lo);
-            }
+            const unsigned long long pk = wave_candidate<T>(hk, lo);
             const int wg = (int)(lo & 1023u);
             if (hk != 0ull && tid == (wg & (kThreads - 1))) {
                 const int tw = wg / kThreads;
@@ -345,15 +365,7 @@ __device__ __forceinline__ void subpanel_factor(cx<T>* __restrict__ P, int m, in
                 hk = better ? k : hk;
                 lo = better ? l : lo;
             }
-            unsigned long long pk = 0;  // complex64: key and position in one word
-            if (sizeof(T) == 4) {
-                pk = (hk << 20) | lo;  // hk < 2^32 for complex64
-                wave_argmax64(pk);
-                hk = pk >> 20;
-                lo = (unsigned)(pk & 0xFFFFFull);
-            } else {
-                wave_argmax_packed(hk, lo);
-            }
+            const unsigned long long pk = wave_candidate<T>(hk, lo);
             const int wg = (int)(lo & 1023u);
             if (hk != 0ull && tid == (wg & (kThreads - 1))) {
                 const int tw = wg / kThreads;
@@ -666,372 +678,247 @@ __device__ __forceinline__ void inpanel_update(cx<T>* __restrict__ P, int m, int
     __syncthreads();
 }
 
-// ---- trailing update after a wide panel ------------------------------------------------------
-// Columns [j0 + jbl, ncol) (the matrix, then right-hand sides), chunks of 16
-// columns dealt to the waves.  P: the factored panel (LDS, ld ldp >= n - j0,
-// logical order); Linv: its inverted 16 x 16 diagonal blocks (ld 16).
-// ASM: first panel, whose trailing entries are assembled from the operators
-// (physical row r, column c of A(w) is element r + c n) instead of loaded.
-// G3: the C update uses the Gauss 3M product (cmfma3) instead of four real
-// products per complex one.
-// LG: the factored columns [j0, j0 + jbl) are read from the slot (logical row
-// r at physical row rmap[r]) instead of the LDS panel, and Linv points to
-// their inverted diagonal blocks in the slot: the deferred update of a
-// two-level step, whose jbl = 16..64 columns were factored as several LDS
-// panels (every 16-block full).
-// NBL > 0: the panel has exactly NBL 16-column blocks (jbl = 16 NBL), known at
-// compile time, so the block loops carry no branches and no unused registers.
-// NOC: U12 only (stored to the slot), no C update (the staged deferred update
-// applies C afterwards).
-template <typename T, bool ASM, bool G3, bool LG, int NBL = 0, bool NOC = false>
-__device__ __forceinline__ void wide_trailing(const SysDesc& sd, double w, double w2, cx<T>* __restrict__ S, int ld,
-                                              const int* rmap, int j0, int jbl, int n, int ncol, const cx<T>* P,
-                                              int ldp, const cx<T>* Linv) {
+// ---- left-looking update of the next columns -------------------------------------------------
+// Columns [j0, j0 + wl) of the factorisation, wl <= 16 NCT, brought up to date with
+// the finished 16-column blocks b = kb0 .. kb1-1: with A the columns (rows in
+// logical order), per block U_b = Linv_b A_b (its block row), then A_t -= L_tb U_b for
+// the row tiles t > b.  The columns stay in the accumulators throughout: row tiles are dealt to
+// the wavefronts (tile kWaves q + wave), a tile's register r of lane li + 16 lg
+// holds row M::row(lg, r), column li.  L_tb is read from the slot straight into MFMA operands,
+// one group of tiles ahead of its use (it does not depend on the chain of
+// the U_b); U_b goes through LDS (ub, two alternating buffers) to every wavefront and to the
+// slot.  The owner of tile b + 1 updates it first and forms U_{b+1} before its other
+// tiles, so one barrier per block carries the chain.
+//
+// Each entry of L is read once per 16 NCT columns and each entry of the matrix is written
+// once.  The right-looking update that this replaces read and wrote the whole
+// trailing matrix per LDS panel (n = 256: 10.2 against 3.5 MB a point in complex128,
+// 4.4 of 5.2 TB/s, its bound).
+//
+// from_slot: the columns' current values are in the slot (partly updated, or
+// right-hand sides, j0 >= n), else A(w) is assembled from the operators.  Afterwards the rows
+// from kb1 * 16 on go to the LDS panel P (ld ldp, the first wp columns, padded with zeros
+// to a multiple of 16) and to the slot (the columns from wp on).
+// G3: Gauss 3M products (three accumulators, converted at the ends).
+constexpr int kPB = 8;  // panel columns loaded per batch
+
+template <typename T, int MAXR, int NCT, bool G3>
+__device__ __forceinline__ void left_update(const SysDesc& sd, double w, double w2, cx<T>* __restrict__ S,
+                                            const cx<T>* __restrict__ Lg, int n, const int* rmap, int j0, int wl,
+                                            int kb0, int kb1, bool from_slot, bool whole, cx<T>* P, int ldp, int wp) {
     using M = Mfma<T>;
     using acc_t = typename M::acc;
-    constexpr int NB = NBL ? NBL : WideCfg<T>::NB;
-    if (NBL) jbl = kSB * NBL;
-    // the assembling variant keeps half the C tile (its FP64 operator loads need the registers)
-    constexpr int TA = ASM ? (WideCfg<T>::TA > 2 ? 2 : WideCfg<T>::TA) : WideCfg<T>::TA;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NRT = 4 * MAXR / kWaves;       // row tiles per wavefront
+    constexpr int NR = NRT < 4 ? NRT : 4;        // operand buffers: L is loaded NR tiles ahead
+    constexpr int UL = 17;                       // leading dimension of a U block in LDS
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    const int c0 = j0 + jbl, m2 = n - c0;
-    const int nbl = (jbl + kSB - 1) / kSB;
-    const int nch = (ncol - c0 + kSB - 1) / kSB;
-    // LG: physical rows of this lane's row li in each 16-row block of L11
-    int plr[LG ? NB : 1];
+    const int ntile = (n + kSB - 1) / kSB;
+    cx<T>* ub = P;  // the panel region is free until the end
+    int plr[NRT];   // physical row of row li of each tile
+    acc_t cr[NRT][NCT], ci[NRT][NCT], cy[G3 ? NRT : 1][NCT];
+    // ---- the first operands of the blocks, in flight while the columns are read
 #pragma unroll
-    for (int b = 0; b < (LG ? NB : 1); ++b) plr[b] = LG ? lds1<3>(rmap + j0 + min(kSB * b + li, jbl - 1)) : 0;
-    auto ldL = [&](const cx<T>* p) -> cx<T> { return LG ? ldc<1>(p) : ldc<3>(p); };
-    // element (physical row prow, column col) of the trailing matrix: the
-    // matrix part assembled from the operators at the first panel (ASM), the
-    // right-hand-side columns (col >= n) from the slot; no branch around the loads
-    auto load_el = [&](int prow, int col) -> cx<T> {
-        if (!ASM) return ldc<1>(S + (prow + (size_t)col * ld));
-        const cx<T> a = to_t<T>(assemble_at(sd, (size_t)prow + (size_t)min(col, n - 1) * ld, w, w2));
-        const cx<T> f = ldc<1>(S + (prow + (size_t)max(col, n) * ld));
-        return col < n ? a : f;
+    for (int q = 0; q < NRT; ++q) plr[q] = lds1<3>(rmap + min(kSB * (wave + kWaves * q) + li, n - 1));
+    cx<T> lb[NR][4];  // L_tb operands: [buffer][k-step]
+    auto load_l = [&](int b, int q, int pr, cx<T> (&l)[4]) {
+        const int t = wave + kWaves * q;
+        if (t > b && t < ntile)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) l[k] = ldc<1>(S + (pr + (size_t)(kSB * b + M::row(lg, k)) * n));
     };
-    for (int ch = wave; ch < nch; ch += kWaves) {
-        const int cb = c0 + ch * kSB, cw = min(kSB, ncol - cb);
-        // ---- A12 in operand layout: block b, register r = logical row j0 + 16 b + row(lg, r)
-        acc_t are[NB], aim[NB];
+    // the inverted diagonal block of this wavefront's next tile in the chain; zero beyond a
+    // narrow last block (stored with its own width as leading dimension)
+    cx<T> linv[4];
+    int tl = wave;
+    while (tl < kb0) tl += kWaves;
+    auto load_linv = [&]() {
+        if (tl < kb1) {
+            const int kb = min(kSB, n - kSB * tl);
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int k = kSB * b + M::row(lg, r);
-                // rows beyond the panel must be zero (they meet the zeroed panel columns
-                // of L11 and Linv); columns beyond cw only feed unstored results
-                const cx<T> v = load_el(lds1<3>(rmap + j0 + min(k, jbl - 1)), cb + min(li, cw - 1));
-                const bool ok = b < nbl && k < jbl;
-                are[b][r] = ok ? v.re : T(0);
-                aim[b][r] = ok ? v.im : T(0);
-            }
-        // ---- U12 = L11^{-1} A12, block forward substitution
-        acc_t ure[NB], uim[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            acc_zero<T>(ure[b]);
-            acc_zero<T>(uim[b]);
-            if (b < nbl) {
-#pragma unroll
-                for (int a = 0; a < b; ++a) {
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const int k = kSB * a + M::row(lg, s);
-                        const int row = kSB * b + li;
-                        // rows beyond: unstored
-                        cx<T> l = LG ? ldc<1>(S + (plr[b] + (size_t)(j0 + k) * ld))
-                                     : ldc<3>(P + (min(row, jbl - 1) + (size_t)k * ldp));
-                        l.re = -l.re;
-                        l.im = -l.im;
-                        cmfma<T>(are[b], aim[b], l, ure[a][s], uim[a][s]);
-                    }
-                }
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const cx<T> li_v = ldL(Linv + (kSB * kSB * b + li + M::row(lg, s) * kSB));
-                    cmfma<T>(ure[b], uim[b], li_v, are[b][s], aim[b][s]);
-                }
+            for (int k = 0; k < 4; ++k) {
+                const int kk = M::row(lg, k);
+                linv[k] = ldz<1>(Lg + ((size_t)tl * kSB * kSB + min(li, kb - 1) + min(kk, kb - 1) * kb), li < kb && kk < kb);
             }
         }
-        // ---- U12 to the slot
+    };
+    if (kb1 > kb0) {
+        load_linv();
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
+        for (int q = 0; q < NR; ++q) load_l(kb0, q, plr[q], lb[q]);
+    }
+    // ---- the columns as they stand, read along the rows (coalesced) into LDS, all at
+    // once where the region holds them (whole), else 16 at a time, and from there into the tiles
+    const int ldn = n | 1, rb = kSB * kb0, nr = n - rb;
+    static_for([&](auto cc) {
+        constexpr int c = decltype(cc)::value;
+#pragma unroll
+        for (int q = 0; q < NRT; ++q) {
+            acc_zero<T>(cr[q][c]);
+            acc_zero<T>(ci[q][c]);
+        }
+        if (kSB * c < wl) {
+            if (c == 0 || !whole) {
+                const int nc = min(whole ? kSB * NCT : kSB, wl - kSB * c), nbat = (nc + kPB - 1) / kPB;
+                auto fill = [&](auto&& entry) {
+                    for (int e = tid; e < nr * nbat; e += kThreads) {
+                        const int r = rb + e % nr, cb = e / nr * kPB;
+                        const int pr = lds1<3>(rmap + r);
+                        cx<T> v[kPB];
+#pragma unroll
+                        for (int u = 0; u < kPB; ++u) v[u] = entry(pr + (size_t)(j0 + kSB * c + min(cb + u, nc - 1)) * n);
+#pragma unroll
+                        for (int u = 0; u < kPB; ++u)
+                            if (cb + u < nc) stc<3>(P + (r + (cb + u) * ldn), v[u]);
+                    }
+                };
+                if (c) __syncthreads();
+                if (from_slot)
+                    fill([&](size_t e) { return ldc<1>(S + e); });
+                else
+                    with_kind(sd, [&](auto kc) { fill([&](size_t e) { return to_t<T>(elem_at<decltype(kc)::value>(sd, e, w, w2)); }); });
+                __syncthreads();
+            }
+            const cx<T>* pt = P + (whole ? kSB * c * ldn : 0);
+#pragma unroll
+            for (int q = 0; q < NRT; ++q) {
+                const int t = wave + kWaves * q;
+                if (t < ntile && t >= kb0)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const cx<T> v = ldc<3>(pt + (min(kSB * t + M::row(lg, r), n - 1) + min(li, wl - kSB * c - 1) * ldn));
+                        cr[q][c][r] = v.re;
+                        ci[q][c][r] = v.im;
+                    }
+            }
+        }
+    }, std::make_integer_sequence<int, NCT>{});
+    __syncthreads();  // the region's next use: U blocks, or the panel
+    if (kb1 > kb0) {
+        // Gauss form: x = cr (starts at d_r), y = cy (0), z = ci (d_r + d_i)
+        auto to_gauss = [&](int q, int c) {
+            acc_zero<T>(cy[G3 ? q : 0][c]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ci[q][c][r] += cr[q][c][r];
+        };
+        auto from_gauss = [&](int q, int c) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int k = kSB * b + M::row(lg, r);
-                if (b < nbl && k < jbl && li < cw)
-                    stc<1>(S + (lds1<3>(rmap + j0 + k) + (size_t)(cb + li) * ld), cmk<T>(ure[b][r], uim[b][r]));
-            }
-        if (NOC || m2 <= 0) continue;
-        // ---- C -= L21 U12, transposed: D = U12^T L21^T; register r of tile a holds
-        // C[row 16 a + li][column row(lg, r)]
-        __builtin_amdgcn_wave_barrier();
-        auto load_c = [&](int r0, acc_t (&cre)[TA], acc_t (&cim)[TA], int (&pr)[TA]) {
-#pragma unroll
-            for (int a = 0; a < TA; ++a) {
-                const int row = r0 + kSB * a + li;
-                pr[a] = lds1<3>(rmap + c0 + min(row, m2 - 1));
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int col = M::row(lg, r);
-                    // rows beyond m2 and columns beyond cw are computed but never stored
-                    const cx<T> v = load_el(pr[a], cb + min(col, cw - 1));
-                    cre[a][r] = v.re;
-                    cim[a][r] = v.im;
-                }
+                const T x = cr[q][c][r], y = cy[G3 ? q : 0][c][r];
+                cr[q][c][r] = x - y;
+                ci[q][c][r] = ci[q][c][r] - x - y;
             }
         };
-        acc_t cre[TA], cim[TA];
-        acc_t cy[G3 ? TA : 1];  // G3: sum of a_i b_i
-        int prow[TA];
-        load_c(0, cre, cim, prow);
-        for (int r0 = 0; r0 < m2; r0 += kSB * TA) {
-            acc_t nre[TA], nim[TA];
-            int nprow[TA];
-            const bool more = r0 + kSB * TA < m2;
-            if (more && !ASM) load_c(r0 + kSB * TA, nre, nim, nprow);
-            if (G3) {
+        if (G3)
 #pragma unroll
-                for (int a = 0; a < TA; ++a) {
-                    acc_zero<T>(cy[a]);
+            for (int q = 0; q < NRT; ++q)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) cim[a][r] += cre[a][r];
-                }
+                for (int c = 0; c < NCT; ++c) to_gauss(q, c);
+        // U_t = Linv_t A_t of tile q into its LDS buffer
+        auto make_u = [&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            cx<T>* u = ub + (tl & 1) * NCT * kSB * UL;
+#pragma unroll
+            for (int c = 0; c < NCT; ++c) {
+                if (G3) from_gauss(q, c);
+                acc_t ur, ui;
+                acc_zero<T>(ur);
+                acc_zero<T>(ui);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) cmfma<T>(ur, ui, linv[k], cr[q][c][k], ci[q][c][k]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) stc<3>(u + ((kSB * c + li) * UL + M::row(lg, r)), cmk<T>(ur[r], ui[r]));
             }
+            tl += kWaves;
+            load_linv();
+        };
+        static_for([&](auto qc) {
+            if (wave + kWaves * decltype(qc)::value == kb0) make_u(qc);
+        }, std::make_integer_sequence<int, NRT>{});
+        __syncthreads();
+        for (int b = kb0; b < kb1; ++b) {
+            const cx<T>* u = ub + (b & 1) * NCT * kSB * UL;
+            T vr[NCT][4], vi[NCT][4];
 #pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                if (b < nbl) {
+            for (int c = 0; c < NCT; ++c)
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const int k = kSB * b + M::row(lg, s);
-                        // A operand: -U12^T (lane: U12[k][li], zero for k beyond the panel, whose
-                        // LDS columns up to the next multiple of 16 are zero)
-                        const cx<T> ua = cmk<T>(-ure[b][s], -uim[b][s]);
-                        cx<T> lv[TA];
+                for (int k = 0; k < 4; ++k) {
+                    const cx<T> v = ldc<3>(u + ((kSB * c + li) * UL + M::row(lg, k)));
+                    vr[c][k] = v.re;
+                    vi[c][k] = v.im;
+                }
+            // U_b to the slot, 16 rows of a column together
+            for (int e = tid; e < kSB * wl; e += kThreads) {
+                const int r = e & (kSB - 1), c = e / kSB;
+                if (kSB * b + r < n)
+                    stc<1>(S + (lds1<3>(rmap + kSB * b + r) + (size_t)(j0 + c) * n), ldc<3>(u + (c * UL + r)));
+            }
+            static_for([&](auto qc) {
+                constexpr int q = decltype(qc)::value, lq = (q + NR) % NRT;
+                const int t = wave + kWaves * q;
+                if (t > b && t < ntile) {
 #pragma unroll
-                        for (int a = 0; a < TA; ++a) {
-                            const int row = min(r0 + kSB * a + li, m2 - 1);
-                            // LG: L21 shares its physical rows with the C tile
-                            lv[a] = LG ? ldc<1>(S + (prow[a] + (size_t)(j0 + k) * ld))
-                                       : ldc<3>(P + ((jbl + row) + (size_t)k * ldp));
-                        }
+                    for (int k = 0; k < 4; ++k) {
+                        const cx<T> l = cmk<T>(-lb[q % NR][k].re, -lb[q % NR][k].im);
                         if (G3) {
-                            const T us = -(ure[b][s] + uim[b][s]);
+                            const T ls = l.re + l.im;
 #pragma unroll
-                            for (int a = 0; a < TA; ++a)
-                                cmfma3<T>(cre[a], cy[a], cim[a], ua, us, lv[a].re, lv[a].im);
+                            for (int c = 0; c < NCT; ++c)
+                                cmfma3<T>(cr[q][c], cy[G3 ? q : 0][c], ci[q][c], l, ls, vr[c][k], vi[c][k]);
                         } else {
 #pragma unroll
-                            for (int a = 0; a < TA; ++a) cmfma<T>(cre[a], cim[a], ua, lv[a].re, lv[a].im);
+                            for (int c = 0; c < NCT; ++c) cmfma<T>(cr[q][c], ci[q][c], l, vr[c][k], vi[c][k]);
                         }
                     }
                 }
-            }
-            if (G3) {
-#pragma unroll
-                for (int a = 0; a < TA; ++a)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const T x = cre[a][r], y = cy[a][r];
-                        cre[a][r] = x - y;
-                        cim[a][r] = cim[a][r] - x - y;
-                    }
-            }
-#pragma unroll
-            for (int a = 0; a < TA; ++a) {
-                const int row = r0 + kSB * a + li;
-                if (row < m2) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int col = M::row(lg, r);
-                        if (col < cw) stc<1>(S + (prow[a] + (size_t)(cb + col) * ld), cmk<T>(cre[a][r], cim[a][r]));
-                    }
-                }
-            }
-            if (more) {
-                if (ASM) {
-                    load_c(r0 + kSB * TA, cre, cim, prow);
-                } else {
-#pragma unroll
-                    for (int a = 0; a < TA; ++a) {
-                        cre[a] = nre[a];
-                        cim[a] = nim[a];
-                        prow[a] = nprow[a];
-                    }
-                }
-            }
+                // the buffer's next use: NR tiles on, of this block or the next
+                const int bn = q + NR < NRT ? b : b + 1;
+                if (bn < kb1) load_l(bn, lq, plr[lq], lb[q % NR]);
+                if (t == b + 1 && t < ntile && b + 1 < kb1) make_u(qc);
+            }, std::make_integer_sequence<int, NRT>{});
+            __syncthreads();
         }
-        __builtin_amdgcn_wave_barrier();
+        if (G3)
+#pragma unroll
+            for (int q = 0; q < NRT; ++q)
+                if (wave + kWaves * q >= kb1)
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c) from_gauss(q, c);
     }
-}
-
-// ---- deferred update of a two-level step, L21 staged through LDS -------------------------------
-// Columns [c0, ncol) with c0 = j0 + jo, rows [c0, n): C -= L21 U12 where the
-// step's columns [j0, j0 + jo) are factored in the slot.  U12 = L11^{-1} A12 is
-// computed per chunk first (wide_trailing without its C update); then, per
-// band of BR rows, the band's L21 (BR x jo) is staged in the LDS region Pb
-// (pcap complex elements, free between panels, odd leading dimension) and
-// every wavefront updates its chunks' C tiles of the band with U12 read back
-// from the slot.  Each C tile is read and written once per step instead of
-// once per LDS panel, and L21 is read once.  Needs pcap >= 17 jo.
-template <typename T, bool ASM, bool G3>
-__device__ __forceinline__ void wide_trailing_staged(const SysDesc& sd, double w, double w2, cx<T>* __restrict__ S,
-                                                     int ld, const int* rmap, int j0, int jo, int n, int ncol,
-                                                     cx<T>* Pb, long long pcap, const cx<T>* Linv) {
-    using M = Mfma<T>;
-    using acc_t = typename M::acc;
-    constexpr int NB = WideCfg<T>::NB;
-    constexpr int TA = ASM ? (WideCfg<T>::TA > 2 ? 2 : WideCfg<T>::TA) : WideCfg<T>::TA;
-    wide_trailing<T, ASM, G3, true, 0, true>(sd, w, w2, S, ld, rmap, j0, jo, n, ncol, Pb, 0, Linv);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int li = lane & 15, lg = lane >> 4;
-    const int c0 = j0 + jo, m2 = n - c0;
-    const int nbl = jo / kSB;
-    const int nch = (ncol - c0 + kSB - 1) / kSB;
-    if (m2 <= 0) return;
-    // band height: a multiple of 64 rows when one fits, else of 16 (the tile
-    // loop clamps a partial band)
-    int BR = (int)(pcap / jo) / 16 * 16;
-    if (BR >= 64) BR = BR / 64 * 64;
-    while (BR > 16 && (long long)(BR | 1) * jo > pcap) BR -= (BR > 64 ? 64 : 16);
-    const int ldb = BR | 1;
-    auto load_el = [&](int prow, int col) -> cx<T> {
-        if (!ASM) return ldc<1>(S + (prow + (size_t)col * ld));
-        const cx<T> a = to_t<T>(assemble_at(sd, (size_t)prow + (size_t)min(col, n - 1) * ld, w, w2));
-        const cx<T> f = ldc<1>(S + (prow + (size_t)max(col, n) * ld));
-        return col < n ? a : f;
-    };
-    for (int rb = 0; rb < m2; rb += BR) {
-        const int nr = min(BR, m2 - rb);
-        __syncthreads();  // U12 stored, the previous band consumed
-        for (int e = tid; e < nr * jo; e += kThreads) {
-            const int r = e % nr, k = e / nr;
-            stc<3>(Pb + (r + (size_t)k * ldb), ldc<1>(S + (lds1<3>(rmap + c0 + rb + r) + (size_t)(j0 + k) * ld)));
-        }
-        __syncthreads();
-        for (int ch = wave; ch < nch; ch += kWaves) {
-            const int cb = c0 + ch * kSB, cw = min(kSB, ncol - cb);
-            // U12 of the chunk back from the slot, operand layout (lane: U12[k][li])
-            acc_t ure[NB], uim[NB];
+    // ---- the updated rows to the LDS panel and to the slot
+    const int r0 = kSB * kb1;
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
+    for (int q = 0; q < NRT; ++q) {
+        const int t = wave + kWaves * q;
+        if (t >= kb1 && t < ntile) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int k = kSB * b + M::row(lg, q);
-                    const cx<T> v = ldc<1>(S + (lds1<3>(rmap + j0 + min(k, jo - 1)) + (size_t)(cb + min(li, cw - 1)) * ld));
-                    const bool ok = b < nbl;
-                    ure[b][q] = ok ? v.re : T(0);
-                    uim[b][q] = ok ? v.im : T(0);
-                }
-            auto load_c = [&](int r0, acc_t (&cre)[TA], acc_t (&cim)[TA], int (&pr)[TA]) {
+            for (int r = 0; r < 4; ++r) {
+                const int row = kSB * t + M::row(lg, r);
+                if (row < n) {
+                    const int pr = lds1<3>(rmap + row);
 #pragma unroll
-                for (int a = 0; a < TA; ++a) {
-                    const int row = rb + min(r0 + kSB * a + li, nr - 1);
-                    pr[a] = lds1<3>(rmap + c0 + row);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const cx<T> v = load_el(pr[a], cb + min(M::row(lg, r), cw - 1));
-                        cre[a][r] = v.re;
-                        cim[a][r] = v.im;
-                    }
-                }
-            };
-            acc_t cre[TA], cim[TA];
-            acc_t cy[G3 ? TA : 1];
-            int prow[TA];
-            load_c(0, cre, cim, prow);
-            for (int r0 = 0; r0 < nr; r0 += kSB * TA) {
-                acc_t nre[TA], nim[TA];
-                int nprow[TA];
-                const bool more = r0 + kSB * TA < nr;
-                if (more && !ASM) load_c(r0 + kSB * TA, nre, nim, nprow);
-                if (G3) {
-#pragma unroll
-                    for (int a = 0; a < TA; ++a) {
-                        acc_zero<T>(cy[a]);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) cim[a][r] += cre[a][r];
-                    }
-                }
-#pragma unroll
-                for (int b = 0; b < NB; ++b) {
-                    if (b < nbl) {
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int k = kSB * b + M::row(lg, q);
-                            const cx<T> ua = cmk<T>(-ure[b][q], -uim[b][q]);
-                            cx<T> lv[TA];
-#pragma unroll
-                            for (int a = 0; a < TA; ++a)
-                                lv[a] = ldc<3>(Pb + (min(r0 + kSB * a + li, nr - 1) + (size_t)k * ldb));
-                            if (G3) {
-                                const T us = -(ure[b][q] + uim[b][q]);
-#pragma unroll
-                                for (int a = 0; a < TA; ++a)
-                                    cmfma3<T>(cre[a], cy[a], cim[a], ua, us, lv[a].re, lv[a].im);
-                            } else {
-#pragma unroll
-                                for (int a = 0; a < TA; ++a) cmfma<T>(cre[a], cim[a], ua, lv[a].re, lv[a].im);
-                            }
-                        }
-                    }
-                }
-                if (G3) {
-#pragma unroll
-                    for (int a = 0; a < TA; ++a)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const T x = cre[a][r], y = cy[a][r];
-                            cre[a][r] = x - y;
-                            cim[a][r] = cim[a][r] - x - y;
-                        }
-                }
-#pragma unroll
-                for (int a = 0; a < TA; ++a) {
-                    if (r0 + kSB * a + li < nr) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int col = M::row(lg, r);
-                            if (col < cw) stc<1>(S + (prow[a] + (size_t)(cb + col) * ld), cmk<T>(cre[a][r], cim[a][r]));
-                        }
-                    }
-                }
-                if (more) {
-                    if (ASM) {
-                        load_c(r0 + kSB * TA, cre, cim, prow);
-                    } else {
-#pragma unroll
-                        for (int a = 0; a < TA; ++a) {
-                            cre[a] = nre[a];
-                            cim[a] = nim[a];
-                            prow[a] = nprow[a];
-                        }
+                    for (int c = 0; c < NCT; ++c) {
+                        const int cc = kSB * c + li;
+                        const cx<T> v = cmk<T>(cr[q][c][r], ci[q][c][r]);
+                        if (kSB * c < wp) stc<3>(P + (row - r0 + (size_t)cc * ldp), cc < wp ? v : czero<T>());
+                        if (cc >= wp && cc < wl) stc<1>(S + (pr + (size_t)(j0 + cc) * n), v);
                     }
                 }
             }
         }
     }
-}
-
-// wide_trailing with the panel's block count fixed at compile time for the
-// common widths (16 and 32 columns).
-template <typename T, bool ASM, bool G3>
-__device__ __forceinline__ void wide_trailing_w(const SysDesc& sd, double w, double w2, cx<T>* __restrict__ S, int ld,
-                                                const int* rmap, int j0, int jbl, int n, int ncol, const cx<T>* P,
-                                                int ldp, const cx<T>* Linv) {
-    if (jbl == kSB) wide_trailing<T, ASM, G3, false, 1>(sd, w, w2, S, ld, rmap, j0, jbl, n, ncol, P, ldp, Linv);
-    else if (jbl == 2 * kSB) wide_trailing<T, ASM, G3, false, 2>(sd, w, w2, S, ld, rmap, j0, jbl, n, ncol, P, ldp, Linv);
-    else wide_trailing<T, ASM, G3, false>(sd, w, w2, S, ld, rmap, j0, jbl, n, ncol, P, ldp, Linv);
 }
 
 // ---- the wide-panel factorisation ------------------------------------------------------------
-// TWO: two-level update (lay.jo columns per step); otherwise one level.
-template <typename T, int MAXR, bool G3, bool TWO>
+// Left-looking in steps of 16 NCT columns (32 complex64, 16 complex128: what the
+// accumulators hold beside the operands), each step one or two LDS panels of jb columns; the
+// first group of right-hand sides last, as columns n .. n + nr - 1.
+template <typename T, int MAXR, bool G3>
 __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w2, cx<T>* __restrict__ S,
                                             const Layout& lay, const Lds& L, int nr) {
+    constexpr int NCT = sizeof(T) == 4 ? 2 : 1;
+    constexpr int W = kSB * NCT;
     const int n = s.n, tid = threadIdx.x;
     const size_t nn = (size_t)n * n;
     const int jb = lay.jb;
@@ -1057,94 +944,49 @@ __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w
     if (tid == 0) L.sc[1] = 0;
     __syncthreads();
 
-    // two-level steps of jo > jb columns: the LDS panels of a step update only
-    // the step's own columns, and the columns right of it get one deferred
-    // rank-jo update with L read back from the slot after the step's last
-    // panel; the step holding the matrix's last columns updates everything
-    // panel by panel.  jo <= jb: one level.
-    const int jo = (TWO && lay.jo > jb) ? lay.jo : jb;
-    for (int J0 = 0; J0 < n; J0 += jo) {
-        const int jend = min(J0 + jo, n);
-        const bool defer = TWO && jo > jb && jend < n;
-        for (int j0 = J0; j0 < jend; j0 += jb) {
-            const int jbl = min(jb, n - j0), m = n - j0;
-            // complex64: odd leading dimension, so the columns an MFMA operand read
-            // spans start in different LDS banks (complex128 elements spread already)
-            const int ldp = sizeof(T) == 4 ? (m | 1) : m;
-            // ---- panel into LDS (logical rows), assembled from the operators at j0 = 0:
-            // items of kPB columns of one row (loads in flight together), spread over
-            // all threads, so short panels keep every thread loading
-            const int nbat = (jbl + kPB - 1) / kPB;
-            for (int e = tid; e < m * nbat; e += kThreads) {
-                const int r = e % m, cb = (e / m) * kPB;
-                const int pr = j0 == 0 ? r : lds1<3>(L.rmap + j0 + r);
-                cx<T> v[kPB];
-#pragma unroll
-                for (int u = 0; u < kPB; ++u) {
-                    const int c = min(cb + u, jbl - 1);
-                    v[u] = j0 == 0 ? to_t<T>(assemble_at(s, (size_t)pr + (size_t)c * n, w, w2))
-                                   : ldc<1>(S + (pr + (size_t)(j0 + c) * n));
-                }
-#pragma unroll
-                for (int u = 0; u < kPB; ++u)
-                    if (cb + u < jbl) stc<3>(P + (r + (size_t)(cb + u) * ldp), v[u]);
-                // columns from jbl to the next multiple of 16 read as zero by the
-                // trailing update's last k-block
-                if (cb == 0)
-                    for (int c = jbl; c < ((jbl + kSB - 1) / kSB) * kSB; ++c) stc<3>(P + (r + (size_t)c * ldp), czero<T>());
+    for (int j0 = 0; j0 < n + (nr > 0 ? 1 : 0);) {
+        const bool rhs = j0 >= n;
+        const int first = j0 / W * W;  // the step's first column
+        const bool cont = !rhs && j0 > first;  // a later panel of the step
+        const int jend = rhs ? n + nr : min(first + W, n);
+        const int jbl = rhs ? 0 : min(jb, jend - j0), m = n - j0;
+        // complex64: odd leading dimension, so the columns an MFMA operand read
+        // spans start in different LDS banks (complex128 elements spread already)
+        const int ldp = sizeof(T) == 4 ? (m | 1) : m;
+        left_update<T, MAXR, NCT, G3>(s, w, w2, S, Lg, n, L.rmap, j0, jend - j0, cont ? (j0 - jb) / kSB : 0,
+                                      rhs ? (int)nblk : j0 / kSB, rhs || cont, jb >= W, P, ldp, jbl);
+        __syncthreads();
+        if (rhs) break;
+        // ---- sub-panels
+        for (int c0 = 0; c0 < jbl; c0 += kSB) {
+            const int sbw = min(kSB, jbl - c0);
+            // the sub-panel's chain of barriers is latency-bound: its waves
+            // take issue priority over the other workgroup's update on the CU
+            // (complex64: +0.6 %; complex128 measured -0.6 % and keeps 0)
+            if (sizeof(T) == 4) __builtin_amdgcn_s_setprio(2);
+            // complex64 sub-panels of at most 64 rows: one wavefront, no
+            // barrier per column (measured at n = 256: +2.3 %; with up to 256
+            // rows in one wavefront its serial rank-1 updates cost about what
+            // the barriers save)
+            bool one_wave = false;
+            if constexpr (sizeof(T) == 4) {
+                one_wave = m - c0 <= 64;
+                if (one_wave) subpanel_factor_1w<1>(P, m, ldp, jbl, c0, sbw, j0, L.ipiv, L.rmap, L.sc, mvl);
             }
+            if (!one_wave) subpanel_factor<T, MAXR>(P, m, ldp, jbl, c0, sbw, j0, L.ipiv, L.rmap, L.sc, cand, mvl);
+            if (sizeof(T) == 4) __builtin_amdgcn_s_setprio(0);
+            invert_unit_lower16<T>(P + c0 + (size_t)c0 * ldp, ldp, sbw, Linv + (size_t)(c0 / kSB) * kSB * kSB,
+                                   Lg + (size_t)((j0 + c0) / kSB) * kSB * kSB);
             __syncthreads();
-            // ---- sub-panels
-            for (int c0 = 0; c0 < jbl; c0 += kSB) {
-                const int sbw = min(kSB, jbl - c0);
-                // the sub-panel's chain of barriers is latency-bound: its waves
-                // take issue priority over the other workgroup's update on the CU
-                // (complex64: +0.6 %; complex128 measured -0.6 % and keeps 0)
-                if (sizeof(T) == 4) __builtin_amdgcn_s_setprio(2);
-                // complex64 sub-panels of at most 64 rows: one wavefront, no
-                // barrier per column (measured at n = 256: +2.3 %; with up to 256
-                // rows in one wavefront its serial rank-1 updates cost about what
-                // the barriers save)
-                bool one_wave = false;
-                if constexpr (sizeof(T) == 4) {
-                    one_wave = m - c0 <= 64;
-                    if (one_wave) subpanel_factor_1w<1>(P, m, ldp, jbl, c0, sbw, j0, L.ipiv, L.rmap, L.sc, mvl);
-                }
-                if (!one_wave) subpanel_factor<T, MAXR>(P, m, ldp, jbl, c0, sbw, j0, L.ipiv, L.rmap, L.sc, cand, mvl);
-                if (sizeof(T) == 4) __builtin_amdgcn_s_setprio(0);
-                invert_unit_lower16<T>(P + c0 + (size_t)c0 * ldp, ldp, sbw, Linv + (size_t)(c0 / kSB) * kSB * kSB,
-                                       Lg + (size_t)((j0 + c0) / kSB) * kSB * kSB);
-                __syncthreads();
-                if (c0 + kSB < jbl) inpanel_update<T>(P, m, ldp, jbl, c0, Linv + (size_t)(c0 / kSB) * kSB * kSB);
-            }
-            // ---- the factored panel to the slot (rows at their physical positions)
-            for (int r = tid; r < m; r += kThreads) {
-                const int pr = lds1<3>(L.rmap + j0 + r);
-                for (int c = 0; c < jbl; ++c) stc<1>(S + (pr + (size_t)(j0 + c) * n), ldc<3>(P + (r + (size_t)c * ldp)));
-            }
-            // ---- trailing columns (only the step's own when deferring)
-            const int tcol = defer ? jend : n + nr;
-            // (the two-level kernel keeps one variant of its narrow within-step update:
-            // less code, fewer spills)
-            if (TWO) {
-                if (j0 == 0) wide_trailing<T, true, G3, false>(s, w, w2, S, n, L.rmap, j0, jbl, n, tcol, P, ldp, Linv);
-                else wide_trailing<T, false, G3, false>(s, w, w2, S, n, L.rmap, j0, jbl, n, tcol, P, ldp, Linv);
-            } else {
-                if (j0 == 0) wide_trailing_w<T, true, G3>(s, w, w2, S, n, L.rmap, j0, jbl, n, tcol, P, ldp, Linv);
-                else wide_trailing_w<T, false, G3>(s, w, w2, S, n, L.rmap, j0, jbl, n, tcol, P, ldp, Linv);
-            }
-            __syncthreads();
+            if (c0 + kSB < jbl) inpanel_update<T>(P, m, ldp, jbl, c0, Linv + (size_t)(c0 / kSB) * kSB * kSB);
         }
-        if (TWO && defer) {
-            // ---- deferred update of columns [jend, n + nr) by the step's jo columns
-            const cx<T>* Lgs = Lg + (size_t)(J0 / kSB) * kSB * kSB;
-            // L21 staged through the panel's LDS region ((n | 1) jb >= 17 jo always:
-            // jb >= 16, jo <= 4 jb, n >= jo)
-            const long long pcap = (long long)(n | 1) * jb;
-            if (J0 == 0) wide_trailing_staged<T, true, G3>(s, w, w2, S, n, L.rmap, J0, jo, n, n + nr, P, pcap, Lgs);
-            else wide_trailing_staged<T, false, G3>(s, w, w2, S, n, L.rmap, J0, jo, n, n + nr, P, pcap, Lgs);
-            __syncthreads();
+        // ---- the factored panel to the slot (rows at their physical positions)
+        for (int r = tid; r < m; r += kThreads) {
+            const int pr = lds1<3>(L.rmap + j0 + r);
+            for (int c = 0; c < jbl; ++c) stc<1>(S + (pr + (size_t)(j0 + c) * n), ldc<3>(P + (r + (size_t)c * ldp)));
         }
+        __syncthreads();
+        j0 += jbl;
     }
     if (sizeof(T) == 4) {
         uinv_blocks(S, n, L.rmap, kSB, Ug);
