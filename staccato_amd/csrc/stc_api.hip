@@ -49,6 +49,34 @@ struct DevBuf {
     U* as() const { return reinterpret_cast<U*>(p); }
 };
 
+// Pinned host memory of a handle through which results return to the caller's arrays
+// (plain memory where pinning fails): at most kStageMax bytes, larger results in pieces.
+constexpr size_t kStageMax = 8 << 20;
+struct HostStage {
+    char* p = nullptr;
+    size_t bytes = 0;
+    bool pinned = false;
+    int ensure(size_t b) {
+        if (b <= bytes) return STC_OK;
+        release();
+        b = std::min(kStageMax, (b + 65535) & ~(size_t)65535);
+        pinned = hipHostMalloc((void**)&p, b, hipHostMallocDefault) == hipSuccess;
+        if (!pinned) {
+            (void)hipGetLastError();
+            p = static_cast<char*>(malloc(b));
+        }
+        if (!p) return STC_ENOMEM;
+        bytes = b;
+        return STC_OK;
+    }
+    void release() {
+        if (p && pinned) (void)hipHostFree(p);
+        else free(p);
+        p = nullptr;
+        bytes = 0;
+    }
+};
+
 struct RomDev {
     int n = 0;
     double eta = 0.0;
@@ -104,6 +132,8 @@ struct stc_ctx {
     std::map<int, RomDev> roms;
     DevBuf scratch, counter;
     LaunchOrder order;
+    HostStage stage;
+    hipEvent_t t0 = nullptr, t1 = nullptr;  // around the launch of a host-memory call
     int live_plans = 0;
     std::map<std::pair<int, int>, Policy> policy;  // (order n, refine) -> policy
     // staging for host-memory calls
@@ -141,6 +171,53 @@ int upload(DevBuf& b, const void* src, size_t bytes, hipStream_t st) {
     int rc = b.ensure(bytes ? bytes : 16);
     if (rc) return rc;
     if (bytes) HIP_TRY(hipMemcpyAsync(b.p, src, bytes, hipMemcpyHostToDevice, st));
+    return STC_OK;
+}
+
+// Rows of a packed device buffer on their way to the caller: `rows` rows of `len` bytes,
+// `spitch` bytes apart in the buffer from offset `off` on, `dpitch` apart at dst.
+struct OutRows {
+    size_t off, len, spitch;
+    char* dst;
+    size_t dpitch, rows;
+};
+
+// Bring `total` bytes of dev to the caller's arrays: through the handle's pinned memory, in
+// two alternating halves when they exceed it, so that the copy of one piece runs while
+// the host distributes the other.  (Through a zeroed vector in pageable memory, one copy for
+// each kind of result, a 1000-point n = 60 sweep with its 0.96 MB of results took 272 us,
+// 80 us of it the kernel; this way 202 us.)
+int fetch(HostStage& hs, const void* dev, size_t total, const OutRows* o, int no, hipStream_t st) {
+    if (!total) return STC_OK;
+    int rc = hs.ensure(std::min(total, kStageMax));
+    if (rc) return rc;
+    const size_t piece = total <= hs.bytes ? total : hs.bytes / 2;
+    auto start = [&](size_t a, int half) {
+        return hipMemcpyAsync(hs.p + half * piece, static_cast<const char*>(dev) + a, std::min(piece, total - a),
+                              hipMemcpyDeviceToHost, st);
+    };
+    HIP_TRY(start(0, 0));
+    int half = 0;
+    for (size_t a = 0; a < total; a += piece, half ^= 1) {
+        HIP_TRY(hipStreamSynchronize(st));
+        const size_t b = std::min(total, a + piece);
+        if (b < total) HIP_TRY(start(b, half ^ 1));
+        const char* src = hs.p + half * piece;
+        for (int q = 0; q < no; ++q) {
+            const OutRows& w = o[q];
+            if (!w.rows || !w.len || b <= w.off) continue;
+            size_t i = a > w.off ? (a - w.off) / w.spitch : 0;
+            if (w.len == w.spitch && w.len == w.dpitch) {  // one run
+                const size_t x = std::max(a, w.off), y = std::min(b, w.off + w.rows * w.len);
+                if (x < y) memcpy(w.dst + (x - w.off), src + (x - a), y - x);
+                continue;
+            }
+            for (; i < w.rows && w.off + i * w.spitch < b; ++i) {
+                const size_t s0 = w.off + i * w.spitch, x = std::max(a, s0), y = std::min(b, s0 + w.len);
+                if (x < y) memcpy(w.dst + i * w.dpitch + (x - s0), src + (x - a), y - x);
+            }
+        }
+    }
     return STC_OK;
 }
 
@@ -495,6 +572,25 @@ __global__ void load_rhs_kernel(const double2* B, int n, int nin, const double2*
 }
 
 // T (p x n, ld p) = transpose of A (n x p, ld n)
+// Sums over the frequencies of the adjoint's per-point values adj (nfreq x nq), points with
+// info > 0 left out: blockIdx.y takes one of gridDim.y consecutive slices, a block 64
+// quantities on four interleaved rows of threads, in a fixed order.
+constexpr int kAdjSlices = 64;
+__global__ void adjoint_sum_kernel(const double* adj, const int* info, int nfreq, int nq, double* sums) {
+    __shared__ double part[4][64];
+    const int k = blockIdx.x * 64 + (threadIdx.x & 63), r = threadIdx.x >> 6;
+    const int f0 = (int)((long long)nfreq * blockIdx.y / gridDim.y);
+    const int f1 = (int)((long long)nfreq * (blockIdx.y + 1) / gridDim.y);
+    double v = 0.0;
+    if (k < nq)
+        for (int f = f0 + r; f < f1; f += 4)
+            if (info[f] <= 0) v += adj[(size_t)f * nq + k];
+    part[r][threadIdx.x & 63] = v;
+    __syncthreads();
+    if (r == 0 && k < nq)
+        sums[(size_t)blockIdx.y * nq + k] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
+}
+
 __global__ void transpose_kernel(const double* A, int n, int p, double* T) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e < n * p) T[e] = A[e / p + (size_t)(e % p) * n];
@@ -541,7 +637,10 @@ int stc_create(stc_handle* out, int device) {
         delete h;
         return STC_ENOMEM;
     }
-    if (hipEventCreateWithFlags(&h->order.ev, hipEventDisableTiming) != hipSuccess) {
+    if (hipEventCreateWithFlags(&h->order.ev, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreate(&h->t0) != hipSuccess || hipEventCreate(&h->t1) != hipSuccess) {
+        for (hipEvent_t e : {h->order.ev, h->t0, h->t1})
+            if (e) (void)hipEventDestroy(e);
         h->counter.release();
         (void)hipStreamDestroy(h->stream);
         delete h;
@@ -561,7 +660,8 @@ int stc_destroy(stc_handle h) {
         DeviceGuard g(h->device);
         h->order.drain();
         (void)hipStreamSynchronize(h->stream);
-        (void)hipEventDestroy(h->order.ev);
+        for (hipEvent_t e : {h->order.ev, h->t0, h->t1}) (void)hipEventDestroy(e);
+        h->stage.release();
         for (auto& kv : h->roms) {
             kv.second.K.release(); kv.second.M.release(); kv.second.D.release();
             kv.second.B.release(); kv.second.C.release();
@@ -766,13 +866,14 @@ int stc_sweep(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int nr
     hipStream_t st = h->stream;
     int rc = upload(h->freq, freq_hz, sizeof(double) * nfreq, st);
     if (rc) return rc;
-    rc = upload_block(h->F, F, n, nrhs, ldf, st);
+    // a packed load needs no second copy, nor the wait for it (the call waits for its results)
+    rc = ldf == n ? upload(h->F, F, sizeof(stc_z64) * (size_t)n * nrhs, st) : upload_block(h->F, F, n, nrhs, ldf, st);
     if (rc) return rc;
     const size_t xcount = (size_t)nfreq * n * nrhs;
-    if ((rc = h->X.ensure(xcount * sizeof(stc_z64)))) return rc;
-    if ((rc = h->info.ensure(sizeof(int) * nfreq))) return rc;
-    if ((rc = h->iters.ensure(sizeof(int) * nfreq))) return rc;
-    if (berr && (rc = h->berr.ensure(sizeof(double) * nfreq * nrhs))) return rc;
+    // X, backward errors, info and iteration counts in one buffer, one copy back
+    const size_t xb = xcount * sizeof(stc_z64), bb = berr ? sizeof(double) * nfreq * nrhs : 0, ib = sizeof(int) * nfreq;
+    if ((rc = h->X.ensure(xb + bb + 2 * ib))) return rc;
+    char* tail = h->X.as<char>() + xb;
 
     const auto& r = it->second;
     KParams kp = base_params(mode, tol, max_iter);
@@ -782,39 +883,31 @@ int stc_sweep(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int nr
     s.freq = h->freq.as<double>();
     s.F = h->F.as<double2>();
     s.X = h->X.as<double2>();
-    s.info = h->info.as<int>();
-    s.berr = berr ? h->berr.as<double>() : nullptr;
-    s.iters = h->iters.as<int>();
+    s.info = reinterpret_cast<int*>(tail + bb);
+    s.berr = berr ? reinterpret_cast<double*>(tail) : nullptr;
+    s.iters = reinterpret_cast<int*>(tail + bb + ib);
     LaunchCfg cfg;
     rc = configure(h, sys, nfreq, mode == STC_REFINED_FP32, 0, &cfg);
     if (rc) return rc;
     kp.one = sys[0];
     kp.nitems = nfreq;
     if (berr) kp.flags |= kWantBerr;
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, st));
+    HIP_TRY(hipEventRecord(h->t0, st));
     rc = enqueue(h, cfg, kp, st);
-    HIP_TRY(hipEventRecord(e1, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (rc) return rc;
-    // copy out (X packed n x nrhs per frequency -> caller's ldx)
-    std::vector<stc_z64> xh(xcount);
-    HIP_TRY(hipMemcpy(xh.data(), h->X.p, xcount * sizeof(stc_z64), hipMemcpyDeviceToHost));
-    for (int f = 0; f < nfreq; ++f)
-        for (int c = 0; c < nrhs; ++c)
-            memcpy(X + ((size_t)f * nrhs + c) * ldx, &xh[((size_t)f * nrhs + c) * n],
-                   sizeof(stc_z64) * n);
-    HIP_TRY(hipMemcpy(info, h->info.p, sizeof(int) * nfreq, hipMemcpyDeviceToHost));
+    HIP_TRY(hipEventRecord(h->t1, st));
+    if (rc) {
+        (void)hipStreamSynchronize(st);
+        return rc;
+    }
     std::vector<int> its(nfreq);
-    HIP_TRY(hipMemcpy(its.data(), h->iters.p, sizeof(int) * nfreq, hipMemcpyDeviceToHost));
-    if (berr)
-        HIP_TRY(hipMemcpy(berr, h->berr.p, sizeof(double) * nfreq * nrhs, hipMemcpyDeviceToHost));
+    const size_t nb = sizeof(stc_z64) * n;
+    const OutRows o[] = {{0, nb, nb, reinterpret_cast<char*>(X), sizeof(stc_z64) * ldx, (size_t)nfreq * nrhs},
+                         {xb, bb, bb, reinterpret_cast<char*>(berr), bb, berr ? (size_t)1 : 0},
+                         {xb + bb, ib, ib, reinterpret_cast<char*>(info), ib, 1},
+                         {xb + bb + ib, ib, ib, reinterpret_cast<char*>(its.data()), ib, 1}};
+    if ((rc = fetch(h->stage, h->X.p, xb + bb + 2 * ib, o, 4, st))) return rc;
+    float ms = 0.f;
+    (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (stats) {
         stats->seconds = ms * 1e-3;
         stats->points = nfreq;
@@ -978,17 +1071,12 @@ int stc_sweep_batch(stc_handle h, int nsys, const stc_sys_desc* sysd, int mode, 
     kp.items = h->items.as<int2>();
     kp.nitems = (int)items.size();
     kp.flags |= kWantBerr;
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, st));
+    HIP_TRY(hipEventRecord(h->t0, st));
     rc = enqueue(h, cfg, kp, st);
-    HIP_TRY(hipEventRecord(e1, st));
+    HIP_TRY(hipEventRecord(h->t1, st));
     HIP_TRY(hipStreamSynchronize(st));
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (rc) return rc;
     std::vector<stc_z64> xh(std::max<size_t>(1, nX));
     std::vector<int> ih(std::max<size_t>(1, nf));
@@ -1133,14 +1221,23 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     hipStream_t st = h->stream;
     int rc;
     if ((rc = upload(h->freq, freq_hz, sizeof(double) * nfreq, st))) return rc;
-    if ((rc = upload_block(h->F, F, n, nrhs, ldf, st))) return rc;
+    if ((rc = ldf == n ? upload(h->F, F, sizeof(stc_z64) * (size_t)n * nrhs, st) : upload_block(h->F, F, n, nrhs, ldf, st)))
+        return rc;
     if ((rc = upload(h->c, c, sizeof(stc_z64) * n, st))) return rc;
-    std::vector<double> ph((size_t)n * std::max(p, 1));
-    for (int k = 0; k < p; ++k) memcpy(&ph[(size_t)k * n], Phi + (size_t)k * ldphi, sizeof(double) * n);
-    if ((rc = upload(h->phi, ph.data(), ph.size() * sizeof(double), st))) return rc;
+    const size_t nph = (size_t)n * std::max(p, 1);
+    std::vector<double> ph;  // Phi packed, unless it is (no mode: zeros)
+    if (p == 0 || ldphi != n) {
+        ph.resize(nph);
+        for (int k = 0; k < p; ++k) memcpy(&ph[(size_t)k * n], Phi + (size_t)k * ldphi, sizeof(double) * n);
+    }
+    if ((rc = upload(h->phi, ph.empty() ? Phi : ph.data(), nph * sizeof(double), st))) return rc;
     if ((rc = upload(h->kd, p ? kdiag : ph.data(), sizeof(double) * std::max(p, 1), st))) return rc;
-    if ((rc = h->adj.ensure(sizeof(double) * (size_t)nfreq * (p + 2)))) return rc;
-    if ((rc = h->info.ensure(sizeof(int) * nfreq))) return rc;
+    // per point {J, dJ/deta, dJ/ds}, then the sums over the slices of the frequencies and info
+    const int nsl = std::min(kAdjSlices, (nfreq + 31) / 32), nq = p + 2;
+    const size_t ab = sizeof(double) * (size_t)nfreq * nq, sb = sizeof(double) * nsl * nq, ib = sizeof(int) * nfreq;
+    if ((rc = h->adj.ensure(ab + sb + ib))) return rc;
+    double* sums = reinterpret_cast<double*>(h->adj.as<char>() + ab);
+    int* dinfo = reinterpret_cast<int*>(h->adj.as<char>() + ab + sb);
     KParams kp = base_params(mode, tol, max_iter);
     kp.flags |= kAdjoint;
     std::vector<SysDesc> sys(1, base_desc(it->second));
@@ -1148,7 +1245,7 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     s.nrhs = nrhs; s.nfreq = nfreq; s.ldf = n; s.ldx = n;
     s.freq = h->freq.as<double>();
     s.F = h->F.as<double2>();
-    s.info = h->info.as<int>();
+    s.info = dinfo;
     s.p = p;
     s.c = h->c.as<double2>();
     s.Phi = h->phi.as<double>();
@@ -1158,7 +1255,7 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     LaunchCfg cfg;
     if ((rc = configure(h, sys, nfreq, refine, 1, &cfg))) return rc;
     if (cfg.wide == kKindRegAdj) {  // reads Phi along its modes
-        if ((rc = h->phiT.ensure(ph.size() * sizeof(double)))) return rc;
+        if ((rc = h->phiT.ensure(nph * sizeof(double)))) return rc;
         const int cnt = n * std::max(p, 1);
         hipLaunchKernelGGL(transpose_kernel, dim3((cnt + 255) / 256), dim3(256), 0, st, h->phi.as<double>(), n,
                            std::max(p, 1), h->phiT.as<double>());
@@ -1168,22 +1265,18 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     kp.one = sys[0];
     kp.nitems = nfreq;
     if ((rc = enqueue(h, cfg, kp, st))) return rc;
-    HIP_TRY(hipStreamSynchronize(st));
-    std::vector<double> ao((size_t)nfreq * (p + 2));
-    HIP_TRY(hipMemcpy(ao.data(), h->adj.p, ao.size() * sizeof(double), hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(info, h->info.p, sizeof(int) * nfreq, hipMemcpyDeviceToHost));
-    double Js = 0.0, Es = 0.0;
-    std::vector<double> ds(std::max(p, 1), 0.0);
-    for (int f = 0; f < nfreq; ++f) {
-        if (info[f] > 0) continue;
-        const double* o = &ao[(size_t)f * (p + 2)];
-        Js += o[0];
-        Es += o[1];
-        for (int k = 0; k < p; ++k) ds[k] += o[2 + k];
-    }
-    *J = Js;
-    *dJ_deta = Es;
-    for (int k = 0; k < p; ++k) dJ_ds[k] = ds[k];
+    hipLaunchKernelGGL(adjoint_sum_kernel, dim3((nq + 63) / 64, nsl), dim3(256), 0, st, h->adj.as<double>(), dinfo,
+                       nfreq, nq, sums);
+    HIP_TRY(hipGetLastError());
+    std::vector<double> sl((size_t)nsl * nq), tot(nq, 0.0);
+    const OutRows o[] = {{0, sb, sb, reinterpret_cast<char*>(sl.data()), sb, 1},
+                         {sb, ib, ib, reinterpret_cast<char*>(info), ib, 1}};
+    if ((rc = fetch(h->stage, sums, sb + ib, o, 2, st))) return rc;
+    for (int q = 0; q < nsl; ++q)
+        for (int k = 0; k < nq; ++k) tot[k] += sl[(size_t)q * nq + k];
+    *J = tot[0];
+    *dJ_deta = tot[1];
+    for (int k = 0; k < p; ++k) dJ_ds[k] = tot[2 + k];
     return status_from_info(info, nfreq, nullptr);
 }
 
@@ -1210,8 +1303,8 @@ int stc_back_transform(stc_handle h, int rom_id, int nfreq, const double* freq_h
     if ((rc = upload(h->freq, freq_hz, sizeof(double) * nfreq, st))) return rc;
     if ((rc = upload(h->load, input_load, sizeof(stc_z64) * (size_t)nin * nrhs, st))) return rc;
     if ((rc = h->F.ensure(sizeof(stc_z64) * (size_t)n * ncol))) return rc;
-    if ((rc = h->info.ensure(sizeof(int) * nfreq))) return rc;
-    if ((rc = h->berr.ensure(sizeof(stc_z64) * (size_t)nfreq * nout * ncol))) return rc;
+    const size_t ycount = (size_t)nfreq * nout * ncol;  // Y and H, then info
+    if ((rc = h->berr.ensure(sizeof(stc_z64) * ycount + sizeof(int) * nfreq))) return rc;
     {
         const long long cnt = (long long)n * ncol;
         hipLaunchKernelGGL(load_rhs_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st,
@@ -1232,30 +1325,22 @@ int stc_back_transform(stc_handle h, int rom_id, int nfreq, const double* freq_h
     s.C = r.C.as<double2>();
     s.Y = Yd;
     s.nout = nout;
-    s.info = h->info.as<int>();
+    s.info = reinterpret_cast<int*>(Yd + ycount);
     LaunchCfg cfg;
     if ((rc = configure(h, sys, nfreq, mode == STC_REFINED_FP32, 0, &cfg))) return rc;
     kp.one = sys[0];
     kp.nitems = nfreq;
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, st));
+    HIP_TRY(hipEventRecord(h->t0, st));
     if ((rc = enqueue(h, cfg, kp, st))) return rc;
-    HIP_TRY(hipEventRecord(e1, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(hipEventRecord(h->t1, st));
+    const size_t yb = sizeof(stc_z64) * nout * nrhs, hb = sizeof(stc_z64) * nout * nin, rb = sizeof(stc_z64) * nout * ncol;
+    const size_t tb = rb * nfreq, ib = sizeof(int) * nfreq;
+    const OutRows o[] = {{0, yb, rb, reinterpret_cast<char*>(Y), yb, (size_t)nfreq},
+                         {yb, hb, rb, reinterpret_cast<char*>(H), hb, H ? (size_t)nfreq : 0},
+                         {tb, ib, ib, reinterpret_cast<char*>(info), ib, 1}};
+    if ((rc = fetch(h->stage, Yd, tb + ib, o, 3, st))) return rc;
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    std::vector<stc_z64> yh((size_t)nfreq * nout * ncol);
-    HIP_TRY(hipMemcpy(yh.data(), Yd, yh.size() * sizeof(stc_z64), hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(info, h->info.p, sizeof(int) * nfreq, hipMemcpyDeviceToHost));
-    for (int f = 0; f < nfreq; ++f) {
-        const stc_z64* yf = &yh[(size_t)f * nout * ncol];
-        memcpy(Y + (size_t)f * nout * nrhs, yf, sizeof(stc_z64) * nout * nrhs);
-        if (H) memcpy(H + (size_t)f * nout * nin, yf + (size_t)nout * nrhs, sizeof(stc_z64) * nout * nin);
-    }
+    (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (stats) {
         stats->seconds = ms * 1e-3;
         stats->points = nfreq;
@@ -1346,20 +1431,15 @@ int stc_gesv_batched(stc_handle h, int n, int batch, const stc_z64* A, int lda, 
             HIP_TRY(hipMemcpy2DAsync(h->F.as<stc_z64>() + j * n * nrhs, sizeof(stc_z64) * n,
                                      B + j * strideB, sizeof(stc_z64) * ldb, sizeof(stc_z64) * n,
                                      nrhs, hipMemcpyHostToDevice, st));
-    hipEvent_t e0, e1;
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, st));
+    HIP_TRY(hipEventRecord(h->t0, st));
     rc = stc_gesv_batched_dev(h, n, batch, h->A.as<stc_z64>(), (long long)nn, nrhs,
                               h->F.as<stc_z64>(), n, strideB ? (long long)n * nrhs : 0,
                               h->X.as<stc_z64>(), n, h->info.as<int>(),
                               berr ? h->berr.as<double>() : nullptr, mode, tol, max_iter, st);
-    HIP_TRY(hipEventRecord(e1, st));
+    HIP_TRY(hipEventRecord(h->t1, st));
     HIP_TRY(hipStreamSynchronize(st));
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (rc) return rc;
     if (ldx == n && strideX == (long long)n * nrhs)
         HIP_TRY(hipMemcpy(X, h->X.p, sizeof(stc_z64) * n * nrhs * batch, hipMemcpyDeviceToHost));
