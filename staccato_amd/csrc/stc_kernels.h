@@ -413,7 +413,13 @@ struct Mfma<double> {
 };
 
 constexpr int kSolveBlock = 32; // diagonal block of the blocked triangular solves
-constexpr int kResRows = 4;     // rows per lane of the residual
+// Rows per lane of the residual; the register-panel kernel, at three workgroups per CU, has no
+// registers for four (n = 256 refined by that kernel, 1024 points: 6.2 ms, with one 4.29).
+#if defined(STC_INST_WIDE) && STC_INST_WIDE == 0
+constexpr int kResRows = 1;
+#else
+constexpr int kResRows = 4;
+#endif
 constexpr int kUw = kUwCols;    // columns of one wave's U12 chunk
 constexpr int kUwLd = kUwLdCols;
 
@@ -1470,24 +1476,26 @@ __device__ void block_sum(double (&vals)[NS], double* red) {
 // the reads of a column batch are in flight together; real operators are loaded a batch
 // ahead.  The wavefronts' partial sums are added one wavefront after the other.  ADJ, whose
 // lanes stand n entries apart, takes one row a lane, all columns and eight of them (one
-// 64-byte piece a lane) per batch.  RC: columns of a batch.  With one
+// 64-byte piece a lane) per batch, and so does the register-panel kernel (kResRows = 1) for two
+// or four columns.  RC: columns of a batch.  With one
 // row a lane and a branch per right-hand side a pass took 148k cycles at n = 256 (two
 // workgroups per CU, refined, 4 right-hand sides) and 97k at n = 144, 112k and 72k now.
 template <bool ADJ, bool RG, int NG, int RC>
 __device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double w2, const double2* bg, int ldb,
                               const z64* bl, const z64* xs, z64* rs, int gc, bool need_anorm,
                               char* sc, int sc_bytes, double& amax) {
-    constexpr int NR = ADJ ? 1 : kResRows, NS = ADJ ? 1 : kWaves;  // NS: shares of the columns
+    constexpr bool ALL = ADJ || kResRows == 1;  // one row a lane, all columns
+    constexpr int NR = ALL ? 1 : kResRows, NS = ALL ? 1 : kWaves;  // NS: shares of the columns
     const int n = __builtin_amdgcn_readfirstlane(s.n), tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int clo = ADJ ? 0 : wave * n / kWaves, chi = ADJ ? n : (wave + 1) * n / kWaves;
+    const int clo = ALL ? 0 : wave * n / kWaves, chi = ALL ? n : (wave + 1) * n / kWaves;
     // the running sums of a row block: rs itself; for residuals in global memory the
     // scratch behind the row sums if it holds a block
     double* asums = reinterpret_cast<double*>(sc);  // min(n, 64 * NR) doubles
     const bool near = RG && sc_bytes >= 64 * NR * (8 + 16 * gc);
     z64* part = RG && near ? reinterpret_cast<z64*>(sc + 64 * NR * 8) : rs;
     const int ldp = near ? 64 * NR : n;
-    for (int r0 = ADJ ? 64 * wave : 0; r0 < n; r0 += ADJ ? 64 * kWaves : 64 * NR) {
+    for (int r0 = ALL ? 64 * wave : 0; r0 < n; r0 += ALL ? 64 * kWaves : 64 * NR) {
         int i[NR];
         z64 acc[NR][NG];
         double asum[NR];
@@ -1571,7 +1579,7 @@ __device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double
         });
         // sums of the shares, one wavefront after the other; the last one adds b
         for (int q = 0; q < NS; ++q) {
-            if (ADJ || wave == q) {
+            if (ALL || wave == q) {
 #pragma unroll
                 for (int t = 0; t < NR; ++t)
                     if (r0 + lane + 64 * t < n) {
@@ -1605,10 +1613,10 @@ __device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double
                             }
                     }
             }
-            if (!ADJ) __syncthreads();
+            if (!ALL) __syncthreads();
         }
     }
-    if (ADJ) __syncthreads();
+    if (ALL) __syncthreads();
 }
 
 template <bool ADJ, bool RG = false>
@@ -1619,9 +1627,9 @@ __device__ __forceinline__ void residual(const SysDesc& s, double w, double w2, 
     gc = __builtin_amdgcn_readfirstlane(gc);
     double amax = 0.0;
     if (ADJ || gc == 1)
-        residual_rows<ADJ, RG, 1, ADJ ? 8 : 2>(s, w, w2, bg, ldb, bl, xs, rs, 1, need_anorm, sc, sc_bytes, amax);
+        residual_rows<ADJ, RG, 1, ADJ ? 8 : kResRows == 1 ? 4 : 2>(s, w, w2, bg, ldb, bl, xs, rs, 1, need_anorm, sc, sc_bytes, amax);
     else
-        residual_rows<ADJ, RG, kMaxGroup, 1>(s, w, w2, bg, ldb, bl, xs, rs, gc, need_anorm, sc, sc_bytes, amax);
+        residual_rows<ADJ, RG, kMaxGroup, kResRows == 1 ? 2 : 1>(s, w, w2, bg, ldb, bl, xs, rs, gc, need_anorm, sc, sc_bytes, amax);
     // pass 2: the norms of the backward error
     double v[kRedSlots];
 #pragma unroll
