@@ -137,7 +137,7 @@ struct stc_ctx {
     int live_plans = 0;
     std::map<std::pair<int, int>, Policy> policy;  // (order n, refine) -> policy
     // staging for host-memory calls
-    DevBuf freq, F, X, info, berr, iters, fac, ipiv, sys, items, adj, c, phi, phiT, kd, A, load;
+    DevBuf freq, F, X, info, berr, fac, ipiv, sys, items, adj, c, phi, phiT, kd, A, load;
 };
 
 struct stc_plan_s {
@@ -667,7 +667,7 @@ int stc_destroy(stc_handle h) {
             kv.second.B.release(); kv.second.C.release();
         }
         DevBuf* bufs[] = {&h->scratch, &h->counter, &h->freq, &h->F, &h->X, &h->info, &h->berr,
-                          &h->iters, &h->fac, &h->ipiv, &h->sys, &h->items, &h->adj, &h->c,
+                          &h->fac, &h->ipiv, &h->sys, &h->items, &h->adj, &h->c,
                           &h->phi, &h->phiT, &h->kd, &h->A, &h->load};
         for (DevBuf* b : bufs) b->release();
         (void)hipStreamDestroy(h->stream);
