@@ -125,19 +125,23 @@ __device__ __forceinline__ void cfma(cx<T>& acc, cx<T> a, cx<T> b) {
 // 1 / z without overflow of |z|^2
 template <typename T>
 __device__ __forceinline__ cx<T> crecip(cx<T> z);
-// 1 / z, complex128: z scaled by a power of two to [1, 2) in its larger part,
+// 1 / z, complex128: z scaled by a power of two to [0.5, 1) in its larger part,
 // one reciprocal of |z|^2 (hardware estimate and two Newton steps).  Smith's
 // form takes three divisions in a chain; same error (2 ulp against 2.5).
+// One infinite part gives zero, as Smith's form does: an entry of A(w) that
+// overflows (a huge mass, say) holds its degree of freedom at rest.
 template <>
 __device__ __forceinline__ cx<double> crecip(cx<double> z) {
-    const double a = fabs(z.re) >= fabs(z.im) ? z.re : z.im;
+    const bool re_big = fabs(z.re) >= fabs(z.im);
+    const double a = re_big ? z.re : z.im, b = re_big ? z.im : z.re;
     const int e = -__builtin_amdgcn_frexp_exp(a);
     const double x = __builtin_amdgcn_ldexp(z.re, e), y = __builtin_amdgcn_ldexp(z.im, e);
     const double q = fma(x, x, y * y);
     double r = __builtin_amdgcn_rcp(q);
     r = fma(fma(-q, r, 1.0), r, r);
     r = fma(fma(-q, r, 1.0), r, r);
-    return cmk<double>(__builtin_amdgcn_ldexp(x * r, e), __builtin_amdgcn_ldexp(-y * r, e));
+    const bool rest = fabs(a) == __builtin_inf() && fabs(b) < __builtin_inf();
+    return cmk<double>(rest ? 0.0 : __builtin_amdgcn_ldexp(x * r, e), rest ? 0.0 : __builtin_amdgcn_ldexp(-y * r, e));
 }
 // complex64 (the factor of the refined mode, whose rounding the FP64
 // refinement absorbs): Smith's scaling with one hardware reciprocal

@@ -1,0 +1,38 @@
+"""Ends of the floating-point range: entries of A(w) and solutions that overflow stay with the
+degrees of freedom they belong to."""
+import numpy as np
+import pytest
+
+from staccato_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+# every factorisation: registers (the column groups), wide panels of one and two workgroups
+# per CU, the register panel
+ORDERS = [5, 33, 64, 80, 128, 129, 200, 257, 513]
+
+
+@pytest.mark.parametrize("at", [0, 2])
+@pytest.mark.parametrize("n", ORDERS)
+def test_overflowing_mass_holds_its_dof(handle, n, at):
+    """A(w) has an infinite diagonal entry: that unknown is zero, the others solve the system
+    without it.  at = 0: a coupled degree of freedom (its pivot is the first); 2: an
+    uncoupled one further on (its row can be no earlier column's pivot)."""
+    rom, rng = synth.modal_rom(n, 300 + n, 0.02)
+    K, M = rom.K.copy(), rom.M.copy()
+    if at:
+        K[at, :] = K[:, at] = M[at, :] = M[:, at] = 0.0
+    M[at, at] = 1e305
+    freq = np.array([40.0, 410.0])
+    F = synth.complex_normal(rng, (n, 3))
+    handle.rom_set(0, K, M, None, rom.eta)
+    X, info, _, _ = handle.sweep(0, freq, F, mode="plain", berr=False)
+    assert (info == 0).all()
+    keep = np.arange(n) != at
+    for j, f in enumerate(freq):
+        A = ((1 + 1j * rom.eta) * K - (2 * np.pi * f) ** 2 * np.where(M > 1e300, 0.0, M))[np.ix_(keep, keep)]
+        ref = np.linalg.solve(A, F[keep])
+        assert (X[j, at] == 0).all()
+        # LU with partial pivoting on both sides: n u each, times the condition number
+        tol = 2 * n * 2.2e-16 * np.linalg.cond(A) * np.sqrt(n) + 1e-14
+        assert np.abs(X[j, keep] - ref).max() <= tol * np.abs(ref).max()
