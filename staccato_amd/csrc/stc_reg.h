@@ -734,12 +734,14 @@ __device__ __forceinline__ void wave_substitute(z64 (&v)[RM], int n, FA&& at, FD
 #pragma unroll
             for (int t = 0; t < RM; ++t) {
                 const int i = lane + 64 * t;
+                // the result is selected, not the coefficient: zero times an unknown that
+                // overflowed would be NaN in the unknowns already found
                 const bool far = BACK ? i < k : i > k;
-                z64 c = la[u][t];
-                c.re = far ? c.re : 0.0;
-                c.im = far ? c.im : 0.0;
+                z64 f = v[t];
+                cfms(f, la[u][t], vk);
                 if (!UNIT && i == k) v[t] = vk;
-                cfms(v[t], c, vk);
+                v[t].re = far ? f.re : v[t].re;
+                v[t].im = far ? f.im : v[t].im;
             }
         }
     };

@@ -36,3 +36,20 @@ def test_overflowing_mass_holds_its_dof(handle, n, at):
         # LU with partial pivoting on both sides: n u each, times the condition number
         tol = 2 * n * 2.2e-16 * np.linalg.cond(A) * np.sqrt(n) + 1e-14
         assert np.abs(X[j, keep] - ref).max() <= tol * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("n", [1, 5, 33, 64, 65, 100, 128, 129, 300])
+def test_overflowing_unknown_leaves_the_others(handle, n):
+    """The first unknown of a diagonal system, found last, overflows: not finite, and the only one."""
+    d = np.full(n, 2.0 + 0j)
+    d[0] = 1e-10
+    B = np.full((n, 2), 1.0 + 0j)
+    B[0, 1] = 1e305
+    X, info, _, _ = handle.gesv_batched(np.diag(d)[None], B, mode="plain", berr=False)
+    assert list(info) == [0]
+    ref = np.full((n, 2), 0.5 + 0j)
+    ref[0] = 1e10
+    assert not np.isfinite(X[0, 0, 1])
+    X[0, 0, 1] = ref[0, 1]
+    # one division each: two roundings
+    np.testing.assert_allclose(X[0], ref, rtol=1e-15, atol=0)
