@@ -111,8 +111,10 @@ int stc_device_ok(stc_handle h);
  * below), 1 = 16-column register panel (three workgroups per CU for
  * complex64, two for complex128), 2 = wide panel held in LDS (up to 32 columns for
  * complex64, 16 for complex128; one or two workgroups per CU, by lds_budget; the
- * automatic choice above n = 128), 3 and 4 = as 2 (they named Gauss 3M products and a
- * two-level update, which 2 has replaced).  lds_budget: bytes of LDS per
+ * automatic choice above n = 128), 3 = as 2 with the complex products of the panels'
+ * update in Gauss 3M form (three real MFMA products instead of four; complex64 up to
+ * n = 256, where it is the automatic choice; other launches run 2), 4 = as 2 (it
+ * named a two-level update that 2 has replaced).  lds_budget: bytes of LDS per
  * workgroup, 0 = automatic, else 16384 .. 163584 (the LDS the panel may use
  * sets the workgroups per CU and the panel width).  jb_max: widest panel
  * (0 = no cap).  An entry applies to launches whose largest system has order

@@ -34,14 +34,19 @@ CANDIDATES = [
     ("wide-2perCU", 2, 80 * 1024, 0),
     ("wide-2perCU-jb16", 2, 80 * 1024, 16),
     ("wide-1perCU", 2, 160 * 1024 - 256, 0),
+    # Gauss 3M complex products in the update of the panels (complex64 only; above
+    # n = 256 the same as kernel 2)
+    ("wide-3M-2perCU", 3, 80 * 1024, 0),
+    ("wide-3M-1perCU", 3, 160 * 1024 - 256, 0),
     # the library's own choice (up to n = 128: systems in registers)
     ("automatic", 0, 0, 0),
 ]
 
 
 def candidates_for(mode):
-    """The candidates of `mode` (the same for both)."""
-    return list(CANDIDATES)
+    """The candidates that differ in `mode` (the 3M kernel exists for complex64 only)."""
+    complex64 = mode in ("refined", "fp32", 1)
+    return [c for c in CANDIDATES if complex64 or c[1] != 3]
 
 
 def default_cache_path():
@@ -88,6 +93,8 @@ def automatic_name(n, mode):
     if n <= 128:
         return "automatic"
     one_per_cu = n > (512 if complex64 else 256)
+    if complex64 and n <= 256:  # Gauss 3M products
+        return "wide-3M-2perCU"
     return "wide-1perCU" if one_per_cu else "wide-2perCU"
 
 

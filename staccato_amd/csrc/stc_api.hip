@@ -113,7 +113,9 @@ struct LaunchOrder {
 }  // namespace
 
 // How the blocked path of a launch runs (stc_policy): kernel 0 = automatic,
-// 1 = 16-column register panel, 2 = wide LDS panel, 3 and 4 = as 2; lds_budget bytes per workgroup (0 = automatic); jb_max caps the panel
+// 1 = 16-column register panel, 2 = wide LDS panel, 3 = wide LDS panel with
+// Gauss 3M products in the update of the panels (complex64 up to n = 256; else as 2),
+// 4 = as 2; lds_budget bytes per workgroup (0 = automatic); jb_max caps the panel
 // width (0 = none).
 struct Policy {
     int kernel = 0;
@@ -332,7 +334,7 @@ Policy policy_for(const stc_ctx* h, int n, int refine) {
 struct LaunchCfg {
     int refine = 0;
     int maxr = 1;
-    int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path;
+    int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path, 2 with 3M products;
                     // reg_kernel: 4, with the adjoint 5
     int threads = kThreads;
     int lds = 0;
@@ -412,7 +414,9 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
     bool blocked = false;
     for (int i = 0; i < nsys; ++i) blocked = blocked || !sys[i].lay_small;
     cfg->wide = 0;
-    if (((pol.kernel == 0 && blocked && maxn > 128) || pol.kernel >= 2) && sweep_kernel_fn(refine, maxr, 1)) {
+    // automatic: Gauss 3M products for complex64 up to n = 256 (built only there)
+    const int wkind = (pol.kernel == 3 || pol.kernel == 0) && sweep_kernel_fn(refine, maxr, 2) ? 2 : 1;
+    if (((pol.kernel == 0 && blocked && maxn > 128) || pol.kernel >= 2) && sweep_kernel_fn(refine, maxr, wkind)) {
         int wcap = wide_jb_max(ts);
         if (pol.jb_max > 0) wcap = std::max(kSB, std::min(pol.jb_max, wcap));
         // automatic LDS budget (measured on MI355X, n = 160 .. 1024): two
@@ -422,7 +426,7 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
         const int budget = pol.lds_budget > 0 ? pol.lds_budget : auto_budget;
         int lds = 0;
         if (layout_wide(sys, nsys, ts, adj, wcap, maxr, budget, &lds)) {  // writes only when all fit
-            cfg->wide = 1;
+            cfg->wide = wkind;
             cfg->lds = lds;
         }
     }

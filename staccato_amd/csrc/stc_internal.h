@@ -19,7 +19,7 @@ namespace stc {
 // was exposed (512 points: n = 1024 refined, 16 right-hand sides 108.4 -> 64.4 ms;
 // n = 512 plain, 4 right-hand sides 12.3 -> 11.0 ms).
 __host__ __device__ constexpr int sweep_threads(int refine, int maxr, int wide) {
-    return wide == 1 && maxr >= (refine ? 16 : 8) ? 512 : 256;
+    return wide >= 1 && wide <= 2 && maxr >= (refine ? 16 : 8) ? 512 : 256;
 }
 #ifdef STC_INST_WIDE
 constexpr int kThreads = sweep_threads(STC_INST_REFINE, STC_INST_MAXR, STC_INST_WIDE);

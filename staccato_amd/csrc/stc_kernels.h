@@ -1924,7 +1924,8 @@ __device__ __forceinline__ void nan_outputs(const SysDesc& s, int fidx) {
 
 // ---- one point ---------------------------------------------------------------------------
 // WIDE != 0: blocked systems use the wide-panel factorisation (factor_wide, LDS
-// panel of lay.jb columns, 16 x 16 inverted diagonal blocks); WIDE == 0: the register panel
+// panel of lay.jb columns, 16 x 16 inverted diagonal blocks), WIDE == 2 with
+// Gauss 3M products in the panels' update; WIDE == 0: the register panel
 // (factor_blocked, lay.jb x lay.jb blocks).
 template <typename T, int MAXR, int WIDE>
 __device__ __forceinline__ void process_point(const SysDesc& s, int fidx, const KParams& kp, char* smem) {
@@ -1971,7 +1972,7 @@ __device__ __forceinline__ void process_point(const SysDesc& s, int fidx, const 
         // right-hand sides eliminated with the factorisation (the first group of
         // a forward sweep)
         const int nr = (kp.flags & (kAdjoint | kFactorOut)) ? 0 : min(nrhs, lay.G);
-        if (WIDE) factor_wide<T, MAXR>(s, w, w2, S, lay, L, nr);
+        if (WIDE) factor_wide<T, MAXR, WIDE == 2>(s, w, w2, S, lay, L, nr);
         else factor_blocked<T, MAXR>(s, w, w2, S, lay, L, nr);
         fused = nr;
         LU = S;

@@ -1,6 +1,7 @@
 // stc_wide.h -- wide-panel blocked LU of the sweep kernel (gfx950).
 //
-// The blocked path of sweep_kernel<T, MAXR, 1>.  It factors A(w) in the workgroup's global factor slot, left-looking,
+// The blocked path of sweep_kernel<T, MAXR, 1> (<T, MAXR, 2>: Gauss 3M products in the
+// panels' update).  It factors A(w) in the workgroup's global factor slot, left-looking,
 // in steps of 32 columns (complex64) or 16 (complex128), with panels of jb columns (a
 // step, or half a complex64 one) held in LDS, one or two workgroups per CU:
 //
@@ -15,7 +16,8 @@
 //   the first right-hand sides are the last step's columns, without a panel.
 //
 // Rows never move in the slot (row map, as in the 16-column path); only the
-// LDS panel is kept in logical order.  Complex products take four real MFMAs.
+// LDS panel is kept in logical order.  Complex products take four real MFMAs
+// (three in the Gauss form).
 //
 // MFMA operand layout used throughout (16x16x4, one wavefront; li = lane % 16,
 // lg = lane / 16): lane supplies A[li][k-slot lg] and B[k-slot lg][li]; the
@@ -35,6 +37,19 @@ __device__ __forceinline__ void cmfma(typename Mfma<T>::acc& dre, typename Mfma<
     dre = M::run(-a.im, bim, dre);
     dim = M::run(a.re, bim, dim);
     dim = M::run(a.im, bre, dim);
+}
+
+// Gauss (3M) form of d += a * b over three accumulators: x += a_r b_r,
+// y += a_i b_i, z += (a_r + a_i)(b_r + b_i); with x, y, z started at (d_r, 0,
+// d_r + d_i) the result is d_r = x - y, d_i = z - x - y.  Three real products
+// instead of four.
+template <typename T>
+__device__ __forceinline__ void cmfma3(typename Mfma<T>::acc& x, typename Mfma<T>::acc& y,
+                                       typename Mfma<T>::acc& z, cx<T> a, T asum, T bre, T bim) {
+    using M = Mfma<T>;
+    x = M::run(a.re, bre, x);
+    y = M::run(a.im, bim, y);
+    z = M::run(asum, bre + bim, z);
 }
 
 template <typename T>
@@ -684,12 +699,10 @@ __device__ __forceinline__ void inpanel_update(cx<T>* __restrict__ P, int m, int
 // right-hand sides, j0 >= n), else A(w) is assembled from the operators.  Afterwards the rows
 // from kb1 * 16 on go to the LDS panel P (ld ldp, the first wp columns, padded with zeros
 // to a multiple of 16) and to the slot (the columns from wp on).
-// Four real products per complex one: Gauss's form with three took no less time (n = 129..256:
-// 0.98..1.01 of it) and its factors were 17 to 21 % less exact, with accumulators converted
-// every 32 columns 13 to 15 %.
+// G3: Gauss 3M products (three accumulators, converted at the ends).
 constexpr int kPB = 8;  // panel columns loaded per batch
 
-template <typename T, int MAXR, int NCT>
+template <typename T, int MAXR, int NCT, bool G3>
 __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double w2, cx<T>* __restrict__ S,
                                             const cx<T>* __restrict__ Lg, int n, const int* rmap, int j0, int wl,
                                             int kb0, int kb1, bool from_slot, bool whole, cx<T>* P, int ldp, int wp) {
@@ -704,7 +717,7 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
     const int ntile = (n + kSB - 1) / kSB;
     cx<T>* ub = P;  // the panel region is free until the end
     int plr[NRT];   // physical row of row li of each tile
-    acc_t cr[NRT][NCT], ci[NRT][NCT];
+    acc_t cr[NRT][NCT], ci[NRT][NCT], cy[G3 ? NRT : 1][NCT];
     // ---- the first operands of the blocks, in flight while the columns are read
 #pragma unroll
     for (int q = 0; q < NRT; ++q) plr[q] = lds1<3>(rmap + min(kSB * (wave + kWaves * q) + li, n - 1));
@@ -783,12 +796,32 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
     }, std::make_integer_sequence<int, NCT>{});
     __syncthreads();  // the region's next use: U blocks, or the panel
     if (kb1 > kb0) {
+        // Gauss form: x = cr (starts at d_r), y = cy (0), z = ci (d_r + d_i)
+        auto to_gauss = [&](int q, int c) {
+            acc_zero<T>(cy[G3 ? q : 0][c]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ci[q][c][r] += cr[q][c][r];
+        };
+        auto from_gauss = [&](int q, int c) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const T x = cr[q][c][r], y = cy[G3 ? q : 0][c][r];
+                cr[q][c][r] = x - y;
+                ci[q][c][r] = ci[q][c][r] - x - y;
+            }
+        };
+        if (G3)
+#pragma unroll
+            for (int q = 0; q < NRT; ++q)
+#pragma unroll
+                for (int c = 0; c < NCT; ++c) to_gauss(q, c);
         // U_t = Linv_t A_t of tile q into its LDS buffer
         auto make_u = [&](auto qc) {
             constexpr int q = decltype(qc)::value;
             cx<T>* u = ub + (tl & 1) * NCT * kSB * UL;
 #pragma unroll
             for (int c = 0; c < NCT; ++c) {
+                if (G3) from_gauss(q, c);
                 acc_t ur, ui;
                 acc_zero<T>(ur);
                 acc_zero<T>(ui);
@@ -828,8 +861,15 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const cx<T> l = cmk<T>(-lb[q % NR][k].re, -lb[q % NR][k].im);
+                        if (G3) {
+                            const T ls = l.re + l.im;
 #pragma unroll
-                        for (int c = 0; c < NCT; ++c) cmfma<T>(cr[q][c], ci[q][c], l, vr[c][k], vi[c][k]);
+                            for (int c = 0; c < NCT; ++c)
+                                cmfma3<T>(cr[q][c], cy[G3 ? q : 0][c], ci[q][c], l, ls, vr[c][k], vi[c][k]);
+                        } else {
+#pragma unroll
+                            for (int c = 0; c < NCT; ++c) cmfma<T>(cr[q][c], ci[q][c], l, vr[c][k], vi[c][k]);
+                        }
                     }
                 }
                 // the buffer's next use: NR tiles on, of this block or the next
@@ -839,6 +879,12 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
             }, std::make_integer_sequence<int, NRT>{});
             __syncthreads();
         }
+        if (G3)
+#pragma unroll
+            for (int q = 0; q < NRT; ++q)
+                if (wave + kWaves * q >= kb1)
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c) from_gauss(q, c);
     }
     // ---- the updated rows to the LDS panel and to the slot
     const int r0 = kSB * kb1;
@@ -868,7 +914,7 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
 // Left-looking in steps of 16 NCT columns (32 complex64, 16 complex128: what the
 // accumulators hold beside the operands), each step one or two LDS panels of jb columns; the
 // first group of right-hand sides last, as columns n .. n + nr - 1.
-template <typename T, int MAXR>
+template <typename T, int MAXR, bool G3>
 __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w2, cx<T>* __restrict__ S,
                                             const Layout& lay, const Lds& L, int nr) {
     constexpr int NCT = sizeof(T) == 4 ? 2 : 1;
@@ -907,7 +953,7 @@ __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w
         // complex64: odd leading dimension, so the columns an MFMA operand read
         // spans start in different LDS banks (complex128 elements spread already)
         const int ldp = sizeof(T) == 4 ? (m | 1) : m;
-        left_update<T, MAXR, NCT>(s, w, w2, S, Lg, n, L.rmap, j0, jend - j0, cont ? (j0 - jb) / kSB : 0,
+        left_update<T, MAXR, NCT, G3>(s, w, w2, S, Lg, n, L.rmap, j0, jend - j0, cont ? (j0 - jb) / kSB : 0,
                                       rhs ? (int)nblk : j0 / kSB, rhs || cont, jb >= W, P, ldp, jbl);
         __syncthreads();
         if (rhs) break;
