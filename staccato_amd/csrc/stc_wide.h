@@ -699,7 +699,12 @@ __device__ __forceinline__ void inpanel_update(cx<T>* __restrict__ P, int m, int
 // right-hand sides, j0 >= n), else A(w) is assembled from the operators.  Afterwards the rows
 // from kb1 * 16 on go to the LDS panel P (ld ldp, the first wp columns, padded with zeros
 // to a multiple of 16) and to the slot (the columns from wp on).
-// G3: Gauss 3M products (three accumulators, converted at the ends).
+// G3: Gauss 3M products (three accumulators, converted at the ends and every 32 finished
+// columns: x and y grow with the columns and cancel in z - x - y.  Converted at the ends only,
+// the factors were 8 % less exact, 41 % at worst, n = 256; the conversions cost 2 %.  Four
+// products take as long as that (n = 129..256: 0.98..1.01) and make factors 11 % more exact,
+// but refined solutions near resonances are less so: at tol 1e-15 the 99.9th percentile of
+// the error against the closed form was 2e-11..1.1e-10, with three 1.1e-11..2e-11.)
 constexpr int kPB = 8;  // panel columns loaded per batch
 
 template <typename T, int MAXR, int NCT, bool G3>
@@ -876,6 +881,12 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
                 const int bn = q + NR < NRT ? b : b + 1;
                 if (bn < kb1) load_l(bn, lq, plr[lq], lb[q % NR]);
                 if (t == b + 1 && t < ntile && b + 1 < kb1) make_u(qc);
+                else if (G3 && (b - kb0) % 2 && b + 1 < kb1 && t > b && t < ntile)
+#pragma unroll
+                    for (int c = 0; c < NCT; ++c) {
+                        from_gauss(q, c);
+                        to_gauss(q, c);
+                    }
             }, std::make_integer_sequence<int, NRT>{});
             __syncthreads();
         }
