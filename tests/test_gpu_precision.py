@@ -38,3 +38,18 @@ def test_factor_error(handle, n):
                 e.append(_factor_error(A, LU[j], ipiv[j] - 1))
                 el.append(_factor_error(A, *sl.lu_factor(A)))
     assert np.mean(e) <= 2.18 * np.mean(el), (np.mean(e), np.mean(el))
+
+
+@pytest.mark.parametrize("n", [320, 512, 1024])
+def test_first_solve_sums(handle, n):
+    """Unrefined solution (tol = 1) of a unit upper triangular system of equal entries c, all
+    unknowns 1: the i-th row from below subtracts c from b_i = 1 + c i, i times.  Summed in blocks of 16
+    first, the n / 16 subtractions round by u times a partial sum that falls from c i to 0,
+    n / 64 u of the backward error's denominator 2 c n, the sums within the blocks by 4.3 u,
+    the rounded load by half a u, the block's inverse by less than 2 u."""
+    c = float(np.float32(0.37))
+    A = np.triu(np.full((n, n), c + 0j), 1) + np.eye(n)
+    b = A @ np.ones((n, 1))
+    _, info, be, _ = handle.gesv_batched(A[None], b, mode="refined", tol=1.0)
+    assert info[0] == 0
+    assert be[0, 0] <= (n / 64 + 7) * 2.0 ** -24, be[0, 0] * 2.0 ** 24
