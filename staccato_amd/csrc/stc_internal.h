@@ -27,11 +27,10 @@ constexpr int kThreads = sweep_threads(STC_INST_REFINE, STC_INST_MAXR, STC_INST_
 constexpr int kThreads = 256;
 #endif
 constexpr int kWaves = kThreads / 64;
-constexpr int kMaxWaves = 8;    // what the LDS layouts allow for
 constexpr int kMaxGroup = 4;    // right-hand sides solved together
 constexpr int kRedSlots = 1 + 5 * kMaxGroup;  // block reductions in the residual
 // reduction scratch: one row of kRedSlots per wave, the result row, scale factors
-constexpr int kRedDoubles = (kMaxWaves + 1) * kRedSlots + kMaxGroup;
+__host__ __device__ constexpr int red_doubles(int waves) { return (waves + 1) * kRedSlots + kMaxGroup; }
 
 // flags of a launch
 enum : int {
@@ -141,9 +140,9 @@ __host__ __device__ inline size_t slot_elems_for(int n, int jb) {
 }
 
 // Fixed region at the start of LDS: ipiv and the row map (n ints each),
-// scalars (16 ints), reduction scratch.
-__host__ __device__ inline int lds_fixed_bytes(int n) {
-    return align16(2LL * n * 4) + align16(16 * 4) + align16((long long)kRedDoubles * 8);
+// scalars (16 ints), reduction scratch.  waves: wavefronts of the kernel that runs.
+__host__ __device__ inline int lds_fixed_bytes(int n, int waves) {
+    return align16(2LL * n * 4) + align16(16 * 4) + align16((long long)red_doubles(waves) * 8);
 }
 
 // Solve vectors: w (factor type), xs, rs (FP64) and, for the adjoint, the
@@ -172,7 +171,7 @@ __host__ __device__ inline long long panel_region_elems(int n, int jb, int maxr)
 // rows per lane of the kernel the launch uses.
 inline Layout plan_layout(int n, int nrhs, int ts, int budget, int jb_cap, int adj, int maxr) {
     Layout L{0, 0, 0, 1, 0};
-    const int fixed = lds_fixed_bytes(n);
+    const int fixed = lds_fixed_bytes(n, sweep_threads(ts == 8, maxr, 0) / 64);
     int Gmax = adj ? 1 : (nrhs < kMaxGroup ? nrhs : kMaxGroup);
     if (Gmax < 1) Gmax = 1;
     for (int G = Gmax; G >= 1; --G) {
@@ -215,14 +214,19 @@ __host__ __device__ constexpr int wide_jb_max(int elem_bytes) { return elem_byte
 
 // LDS of the wide path beyond lds_fixed_bytes: the n x jb panel (leading
 // dimension rounded up to odd, so its columns start in different banks), its inverted
-// 16 x 16 diagonal blocks, the sub-panel's two alternating pivot-candidate
-// buffers (per wave one row of 16 and its 16-byte key) and the moved-row
-// list (2 x 16).  maxr is not needed (kept for the callers' signature).
-__host__ __device__ inline long long wide_cand_bytes(int ts) { return 2LL * kMaxWaves * kSB * ts + 2LL * kMaxWaves * 16; }
-__host__ __device__ inline long long wide_lds_bytes(int n, int jb, int ts, int maxr) {
-    (void)maxr;
-    return align16((long long)(n | 1) * jb * ts) + align16((long long)jb * kSB * ts) + align16(wide_cand_bytes(ts)) +
-           align16(2LL * kSB * 8);
+// 16 x 16 diagonal blocks or, before a block is inverted, the sub-panel's two
+// alternating pivot-candidate buffers (per wave one row of 16 and its 16-byte key), and the
+// moved-row list (2 x 16).  The two alternating U blocks of the left-looking update start
+// where the panel does and are gone before it is written: on a small panel they reach into
+// what follows.
+__host__ __device__ inline int wide_blocks_bytes(int jb, int ts, int waves) {
+    const long long inv = (long long)jb * kSB * ts, cand = 2LL * waves * (kSB * ts + 16);
+    return align16(inv > cand ? inv : cand);
+}
+__host__ __device__ inline long long wide_lds_bytes(int n, int jb, int ts, int waves) {
+    const long long panel = align16((long long)(n | 1) * jb * ts) + wide_blocks_bytes(jb, ts, waves) + align16(2LL * kSB * 8);
+    const long long u = 2LL * wide_jb_max(ts) * (kSB + 1) * ts;
+    return panel > u ? panel : u;
 }
 
 // Layout of a system in a wide-panel launch: the small path when the matrix
@@ -230,7 +234,8 @@ __host__ __device__ inline long long wide_lds_bytes(int n, int jb, int ts, int m
 // jb_cap) that fits.
 inline Layout plan_layout_wide(int n, int nrhs, int ts, int budget, int jb_cap, int adj, int maxr) {
     Layout L{0, 0, 0, 1, 0};
-    const int fixed = lds_fixed_bytes(n);
+    const int waves = sweep_threads(ts == 8, maxr, 1) / 64;
+    const int fixed = lds_fixed_bytes(n, waves);
     int Gmax = adj ? 1 : (nrhs < kMaxGroup ? nrhs : kMaxGroup);
     if (Gmax < 1) Gmax = 1;
     for (int G = Gmax; G >= 1; --G) {
@@ -242,7 +247,7 @@ inline Layout plan_layout_wide(int n, int nrhs, int ts, int budget, int jb_cap, 
     }
     for (int jb = wide_jb_max(ts); jb >= kSB; jb -= kSB) {
         if (jb > jb_cap) continue;
-        const long long need = fixed + wide_lds_bytes(n, jb, ts, maxr);
+        const long long need = fixed + wide_lds_bytes(n, jb, ts, waves);
         if (need <= budget) {
             L.jb = jb; L.cw = kSB; L.lds = (int)need;
             // the largest solve group, with the FP64 residuals in LDS if that

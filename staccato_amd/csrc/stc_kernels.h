@@ -445,7 +445,7 @@ __device__ __forceinline__ Lds carve(char* smem, int n) {
     L.sc = reinterpret_cast<int*>(smem + off);
     off += align16(16 * 4);
     L.red = reinterpret_cast<double*>(smem + off);
-    off += align16((long long)kRedDoubles * 8);
+    off += align16((long long)red_doubles(kWaves) * 8);
     L.main = smem + off;
     return L;
 }

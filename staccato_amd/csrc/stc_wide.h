@@ -720,7 +720,7 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
     const int ntile = (n + kSB - 1) / kSB;
-    cx<T>* ub = P;  // the panel region is free until the end
+    cx<T>* ub = P;  // the panel region and what follows it are free until the end
     int plr[NRT];   // physical row of row li of each tile
     acc_t cr[NRT][NCT], ci[NRT][NCT], cy[G3 ? NRT : 1][NCT];
     // ---- the first operands of the blocks, in flight while the columns are read
@@ -937,9 +937,8 @@ __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w
     cx<T>* P = reinterpret_cast<cx<T>*>(base);
     base += align16((long long)(n | 1) * jb * sizeof(cx<T>));
     cx<T>* Linv = reinterpret_cast<cx<T>*>(base);
-    base += align16((long long)jb * kSB * sizeof(cx<T>));
-    cx<T>* cand = reinterpret_cast<cx<T>*>(base);  // sub-panel pivot candidates
-    base += align16(wide_cand_bytes((int)sizeof(cx<T>)));
+    cx<T>* cand = Linv;  // a sub-panel's pivot candidates, read before any of its blocks is inverted
+    base += wide_blocks_bytes(jb, (int)sizeof(cx<T>), kWaves);
     int2* mvl = reinterpret_cast<int2*>(base);
     const size_t nblk = (size_t)((n + kSB - 1) / kSB);
     cx<T>* Lg = S + (size_t)n * (n + kMaxGroup);

@@ -53,3 +53,19 @@ def test_overflowing_unknown_leaves_the_others(handle, n):
     X[0, 0, 1] = ref[0, 1]
     # one division each: two roundings
     np.testing.assert_allclose(X[0], ref, rtol=1e-15, atol=0)
+
+
+@pytest.mark.parametrize("n,mode,kernel,budget", [(143, "refined", 1, 16384), (230, "refined", 1, 20480),
+                                                  (74, "refined", 2, 16384), (843, "refined", 2, 120000),
+                                                  (29, "plain", 1, 16384), (270, "plain", 1, 32768),
+                                                  (400, "plain", 2, 110000)])
+def test_smallest_lds_budgets(handle, n, mode, kernel, budget):
+    rom, rng = synth.modal_rom(n, 40 + n, 0.02)
+    F = synth.complex_normal(rng, (n, 2))
+    handle.rom_set(0, rom.K, rom.M, rom.D, rom.eta)
+    try:
+        handle.set_policy(n, mode, kernel, budget, 0)
+        _, info, be, _ = handle.sweep(0, [40.0, 410.0, 1300.0], F, mode=mode, tol=1e-12)
+    finally:
+        handle.clear_policies()
+    assert (info == 0).all() and be.max() <= 1e-12
