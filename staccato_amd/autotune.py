@@ -12,8 +12,8 @@ mode.  tune() times every candidate on a sample of the caller's frequencies
 (inputs and outputs resident on the device, HIP events on the launch stream),
 keeps only candidates whose every point meets the tolerance, installs the
 fastest with Handle.set_policy and records it in a JSON cache keyed by
-(arch, n, nrhs, mode).  apply_cached() installs recorded policies without
-measuring.  The reference has no counterpart: its only tuning knob is a fixed
+(arch, n, nrhs, mode).  apply_cached() installs recorded policies of this generation of
+kernels without measuring.  The reference has no counterpart: its only tuning knob is a fixed
 batch size (test/krylovMidsizeTest/gpu/concurrent/batchedLU/src/config/config.cu:29-30).
 """
 import json
@@ -22,6 +22,11 @@ import os
 import numpy as np
 
 ARCH = "gfx950"
+# What the recorded kernel numbers stand for and how fast the automatic choice is
+# beside them; raised when either changes.  Entries of another generation are not installed:
+# they were measured against other kernels ("register-panel", the automatic choice up to
+# n = 128 before the register kernels, would cost 1.2 to 4 times their time).
+GENERATION = 2
 
 # (name, kernel, lds_budget bytes, jb_max)
 CANDIDATES = [
@@ -77,10 +82,10 @@ def save_cache(cache, path=None):
 
 
 def apply_cached(handle, n, nrhs, mode, cache=None):
-    """Install the recorded policy for (n, nrhs, mode); True when one exists."""
+    """Install the recorded policy for (n, nrhs, mode); True when one of this generation exists."""
     cache = load_cache() if cache is None else cache
     e = cache.get(_key(n, nrhs, mode))
-    if not e:
+    if not e or e.get("generation") != GENERATION:
         return False
     handle.set_policy(n, mode, e["kernel"], e["lds_budget"], e["jb_max"])
     return True
@@ -154,6 +159,7 @@ def tune(handle, rom_id, freq_hz, F, mode, tol, sample=1024, reps=3, candidates=
     handle.set_policy(n, mode, best["kernel"], best["lds_budget"], best["jb_max"])
     if cache is not False:
         c = load_cache(cache_path) if cache is None else cache
-        c[_key(n, nrhs, mode)] = {k: best[k] for k in ("name", "kernel", "lds_budget", "jb_max", "pts_per_s")}
+        c[_key(n, nrhs, mode)] = {"generation": GENERATION,
+                                  **{k: best[k] for k in ("name", "kernel", "lds_budget", "jb_max", "pts_per_s")}}
         save_cache(c, cache_path)
     return best, results
