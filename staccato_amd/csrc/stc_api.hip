@@ -174,6 +174,18 @@ int upload(DevBuf& b, const void* src, size_t bytes, hipStream_t st) {
     return STC_OK;
 }
 
+// Copies from the caller's arrays (and the call's own) may be in flight until the stream is
+// waited for, so a call that comes back early waits; settled: it has been.  Declared after the
+// vectors that are copied from.
+struct Uploads {
+    hipStream_t st;
+    bool settled = false;
+    explicit Uploads(hipStream_t s) : st(s) {}
+    ~Uploads() {
+        if (!settled) (void)hipStreamSynchronize(st);
+    }
+};
+
 // Rows of a packed device buffer on their way to the caller: `rows` rows of `len` bytes,
 // `spitch` bytes apart in the buffer from offset `off` on, `dpitch` apart at dst.
 struct OutRows {
@@ -864,6 +876,7 @@ int stc_sweep(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int nr
     if (nfreq == 0) return STC_OK;
     DeviceGuard g(h->device);
     hipStream_t st = h->stream;
+    Uploads up(st);
     int rc = upload(h->freq, freq_hz, sizeof(double) * nfreq, st);
     if (rc) return rc;
     // a packed load needs no second copy, nor the wait for it (the call waits for its results)
@@ -895,10 +908,7 @@ int stc_sweep(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int nr
     HIP_TRY(hipEventRecord(h->t0, st));
     rc = enqueue(h, cfg, kp, st);
     HIP_TRY(hipEventRecord(h->t1, st));
-    if (rc) {
-        (void)hipStreamSynchronize(st);
-        return rc;
-    }
+    if (rc) return rc;
     std::vector<int> its(nfreq);
     const size_t nb = sizeof(stc_z64) * n;
     const OutRows o[] = {{0, nb, nb, reinterpret_cast<char*>(X), sizeof(stc_z64) * ldx, (size_t)nfreq * nrhs},
@@ -906,6 +916,7 @@ int stc_sweep(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int nr
                          {xb + bb, ib, ib, reinterpret_cast<char*>(info), ib, 1},
                          {xb + bb + ib, ib, ib, reinterpret_cast<char*>(its.data()), ib, 1}};
     if ((rc = fetch(h->stage, h->X.p, xb + bb + 2 * ib, o, 4, st))) return rc;
+    up.settled = true;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (stats) {
@@ -934,6 +945,7 @@ int stc_getrf(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int mo
     const size_t ts = refine ? sizeof(stc_c32) : sizeof(stc_z64);
     DeviceGuard g(h->device);
     hipStream_t st = h->stream;
+    Uploads up(st);
     int rc = upload(h->freq, freq_hz, sizeof(double) * nfreq, st);
     if (rc) return rc;
     if ((rc = h->fac.ensure(ts * (size_t)n * n * nfreq))) return rc;
@@ -956,6 +968,7 @@ int stc_getrf(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int mo
     rc = enqueue(h, cfg, kp, st);
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(st));
+    up.settled = true;
     HIP_TRY(hipMemcpy(LU, h->fac.p, ts * (size_t)n * n * nfreq, hipMemcpyDeviceToHost));
     HIP_TRY(hipMemcpy(ipiv, h->ipiv.p, sizeof(int) * (size_t)n * nfreq, hipMemcpyDeviceToHost));
     HIP_TRY(hipMemcpy(info, h->info.p, sizeof(int) * nfreq, hipMemcpyDeviceToHost));
@@ -1040,6 +1053,9 @@ int stc_sweep_batch(stc_handle h, int nsys, const stc_sys_desc* sysd, int mode, 
         ofs_B[i] = cb_;
         cb_ += (size_t)sysd[i].nrhs * sysd[i].nfreq;
     }
+    std::vector<SysDesc> sys;
+    std::vector<int2> items;
+    Uploads up(st);
     int rc;
     if ((rc = upload(h->freq, hf.data(), hf.size() * sizeof(double), st))) return rc;
     if ((rc = upload(h->F, hF.data(), hF.size() * sizeof(stc_z64), st))) return rc;
@@ -1056,8 +1072,6 @@ int stc_sweep_batch(stc_handle h, int nsys, const stc_sys_desc* sysd, int mode, 
         dd[i].info = h->info.as<int>() + ofs_f[i];
         dd[i].berr = sysd[i].berr ? h->berr.as<double>() + ofs_B[i] : nullptr;
     }
-    std::vector<SysDesc> sys;
-    std::vector<int2> items;
     if ((rc = build_batch(h, nsys, dd.data(), sys, items))) return rc;
     if (items.empty()) return STC_OK;
     const bool refine = mode == STC_REFINED_FP32;
@@ -1075,6 +1089,7 @@ int stc_sweep_batch(stc_handle h, int nsys, const stc_sys_desc* sysd, int mode, 
     rc = enqueue(h, cfg, kp, st);
     HIP_TRY(hipEventRecord(h->t1, st));
     HIP_TRY(hipStreamSynchronize(st));
+    up.settled = true;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (rc) return rc;
@@ -1219,13 +1234,14 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     if (ldf < n || (p > 0 && ldphi < n)) return STC_EINVAL;
     DeviceGuard g(h->device);
     hipStream_t st = h->stream;
+    const size_t nph = (size_t)n * std::max(p, 1);
+    std::vector<double> ph;  // Phi packed, unless it is (no mode: zeros)
+    Uploads up(st);
     int rc;
     if ((rc = upload(h->freq, freq_hz, sizeof(double) * nfreq, st))) return rc;
     if ((rc = ldf == n ? upload(h->F, F, sizeof(stc_z64) * (size_t)n * nrhs, st) : upload_block(h->F, F, n, nrhs, ldf, st)))
         return rc;
     if ((rc = upload(h->c, c, sizeof(stc_z64) * n, st))) return rc;
-    const size_t nph = (size_t)n * std::max(p, 1);
-    std::vector<double> ph;  // Phi packed, unless it is (no mode: zeros)
     if (p == 0 || ldphi != n) {
         ph.resize(nph);
         for (int k = 0; k < p; ++k) memcpy(&ph[(size_t)k * n], Phi + (size_t)k * ldphi, sizeof(double) * n);
@@ -1272,6 +1288,7 @@ int stc_adjoint(stc_handle h, int rom_id, int nfreq, const double* freq_hz, int 
     const OutRows o[] = {{0, sb, sb, reinterpret_cast<char*>(sl.data()), sb, 1},
                          {sb, ib, ib, reinterpret_cast<char*>(info), ib, 1}};
     if ((rc = fetch(h->stage, sums, sb + ib, o, 2, st))) return rc;
+    up.settled = true;
     for (int q = 0; q < nsl; ++q)
         for (int k = 0; k < nq; ++k) tot[k] += sl[(size_t)q * nq + k];
     *J = tot[0];
@@ -1296,6 +1313,7 @@ int stc_back_transform(stc_handle h, int rom_id, int nfreq, const double* freq_h
     const int ncol = nrhs + (H ? nin : 0);
     DeviceGuard g(h->device);
     hipStream_t st = h->stream;
+    Uploads up(st);
     int rc;
     // right-hand sides [B_R * inputLoad | B_R] on the device (the projection is
     // frequency independent, hoisted out of the loop of
@@ -1339,6 +1357,7 @@ int stc_back_transform(stc_handle h, int rom_id, int nfreq, const double* freq_h
                          {yb, hb, rb, reinterpret_cast<char*>(H), hb, H ? (size_t)nfreq : 0},
                          {tb, ib, ib, reinterpret_cast<char*>(info), ib, 1}};
     if ((rc = fetch(h->stage, Yd, tb + ib, o, 3, st))) return rc;
+    up.settled = true;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (stats) {
@@ -1408,6 +1427,7 @@ int stc_gesv_batched(stc_handle h, int n, int batch, const stc_z64* A, int lda, 
     DeviceGuard g(h->device);
     hipStream_t st = h->stream;
     const size_t nn = (size_t)n * n, nb = strideB ? (size_t)batch : 1;
+    Uploads up(st);
     int rc;
     if ((rc = h->A.ensure(sizeof(stc_z64) * nn * batch))) return rc;
     if ((rc = h->F.ensure(sizeof(stc_z64) * (size_t)n * nrhs * nb))) return rc;
@@ -1438,6 +1458,7 @@ int stc_gesv_batched(stc_handle h, int n, int batch, const stc_z64* A, int lda, 
                               berr ? h->berr.as<double>() : nullptr, mode, tol, max_iter, st);
     HIP_TRY(hipEventRecord(h->t1, st));
     HIP_TRY(hipStreamSynchronize(st));
+    up.settled = true;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, h->t0, h->t1);
     if (rc) return rc;
