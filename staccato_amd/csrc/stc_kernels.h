@@ -242,9 +242,10 @@ __device__ __forceinline__ z64 assemble_at(const SysDesc& s, size_t e, double w,
 // ---- operator kinds of the assembly (uniform per point) ------------------------------------------
 // The kind is decided around a batch of entries: its branches around each entry would make
 // every load of the batch wait by itself.
-enum : int { kOpReal2 = 0, kOpReal3 = 1, kOpCplx = 2 };
+// kOpOne: an explicit matrix per point (op_stride; no D), one load an entry.
+enum : int { kOpReal2 = 0, kOpReal3 = 1, kOpCplx = 2, kOpOne = 3 };
 __device__ __forceinline__ int op_kind(const SysDesc& s) {
-    return s.real_ops ? (s.has_D ? kOpReal3 : kOpReal2) : kOpCplx;
+    return s.real_ops ? (s.has_D ? kOpReal3 : kOpReal2) : s.op_stride && !s.has_D ? kOpOne : kOpCplx;
 }
 // f(integral_constant<kind>) for the point's kind
 template <typename F>
@@ -252,7 +253,13 @@ __device__ __forceinline__ void with_kind(const SysDesc& s, F&& f) {
     const int k = op_kind(s);
     if (k == kOpReal2) f(std::integral_constant<int, kOpReal2>{});
     else if (k == kOpReal3) f(std::integral_constant<int, kOpReal3>{});
+    else if (k == kOpOne) f(std::integral_constant<int, kOpOne>{});
     else f(std::integral_constant<int, kOpCplx>{});
+}
+// entry k of an explicit matrix (M aliases K; eta and w are zero, so that a part that is not
+// finite makes NaN as in assemble_at)
+__device__ __forceinline__ z64 explicit_at(const SysDesc& s, z64 k, double w2) {
+    return cmk<double>(k.re - s.eta * k.im - w2 * k.re, k.im + s.eta * k.re - w2 * k.im);
 }
 // Entry e of A(w), as assemble_at; explicit matrices (op_stride) read the
 // matrix once (M aliases K there).
@@ -264,6 +271,7 @@ __device__ __forceinline__ z64 elem_at(const SysDesc& s, size_t e, double w, dou
         return cmk<double>(k - w2 * m, s.eta * k + w * d);
     }
     const z64 k = ldc<1>(reinterpret_cast<const z64*>(s.K) + e);
+    if (KIND == kOpOne) return explicit_at(s, k, w2);
     z64 m = k, d = czero<double>();
     if (!s.op_stride) m = ldc<1>(reinterpret_cast<const z64*>(s.M) + e);
     if (s.has_D) d = ldc<1>(reinterpret_cast<const z64*>(s.D) + e);
@@ -1545,6 +1553,7 @@ __device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double
                 }
             } else {
                 double kv[2][RC][NR], mv[2][RC][NR], dv[2][RC][NR];
+                z64 zv[2][RC][NR];
                 auto load = [&](int j0, auto bc) {
                     constexpr int B = decltype(bc)::value;
 #pragma unroll
@@ -1553,9 +1562,13 @@ __device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double
 #pragma unroll
                         for (int t = 0; t < NR; ++t) {
                             const int e = ADJ ? c + i[t] * n : i[t] + c * n;
-                            kv[B][u][t] = lds1<1>(s.K + e);
-                            mv[B][u][t] = lds1<1>(s.M + e);
-                            dv[B][u][t] = KIND == kOpReal3 ? lds1<1>(s.D + e) : 0.0;
+                            if constexpr (KIND == kOpOne) {
+                                zv[B][u][t] = ldc<1>(reinterpret_cast<const z64*>(s.K) + e);
+                            } else {
+                                kv[B][u][t] = lds1<1>(s.K + e);
+                                mv[B][u][t] = lds1<1>(s.M + e);
+                                dv[B][u][t] = KIND == kOpReal3 ? lds1<1>(s.D + e) : 0.0;
+                            }
                         }
                     }
                 };
@@ -1568,8 +1581,13 @@ __device__ __forceinline__ void residual_rows(const SysDesc& s, double w, double
                             solution(j0 + u, x);
 #pragma unroll
                             for (int t = 0; t < NR; ++t)
-                                a[t] = cmk<double>(kv[B][u][t] - w2 * mv[B][u][t],
-                                                   (ADJ ? -1.0 : 1.0) * (s.eta * kv[B][u][t] + w * dv[B][u][t]));
+                                if constexpr (KIND == kOpOne) {
+                                    const z64 e = explicit_at(s, zv[B][u][t], w2);
+                                    a[t] = ADJ ? cconj(e) : e;
+                                } else {
+                                    a[t] = cmk<double>(kv[B][u][t] - w2 * mv[B][u][t],
+                                                       (ADJ ? -1.0 : 1.0) * (s.eta * kv[B][u][t] + w * dv[B][u][t]));
+                                }
                             column(a, x);
                         }
                 };

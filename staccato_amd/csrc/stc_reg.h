@@ -487,7 +487,7 @@ __device__ __forceinline__ void reg_point_refined(const SysDesc* sp, int fidx, c
         const double w = s.freq ? kTwoPi * s.freq[fidx] : 0.0, w2 = w * w;
         with_kind(s, [&](auto kc) {
             constexpr int KIND = decltype(kc)::value;
-            constexpr int QC = RM == 1 ? 4 : 2;
+            constexpr int QC = RM == 1 || KIND == kOpOne ? 4 : 2;
 #pragma unroll
             for (int qc = 0; qc < CPW; qc += QC) {
                 z64 a[QC][RM];
@@ -638,7 +638,7 @@ __device__ __forceinline__ void reg_point_refined(const SysDesc* sp, int fidx, c
                 for (int g = 0; g < G; ++g) ra[t][g] = czero<double>();
             with_kind(s, [&](auto kc) {
                 constexpr int KIND = decltype(kc)::value;
-                constexpr int QC = RM == 1 ? 4 : 2;
+                constexpr int QC = RM == 1 || KIND == kOpOne ? 4 : 2;
                 for (int c0 = QC * wave; c0 < n; c0 += NW * QC) {
                     z64 a[QC][RM];
 #pragma unroll
