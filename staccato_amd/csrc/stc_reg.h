@@ -763,9 +763,148 @@ __device__ __forceinline__ double wave_dsum(double v) {
     return v;
 }
 
+// ---- backward errors of solutions in registers and (vec, [wavefront][n]) in LDS ---------------------
+// Right-hand side g by this wavefront alone: r = F - A(w) x and the row sums of |A|.
+template <int RM>
+__device__ __forceinline__ void reg_berr_wave(const SysDesc& s, int fidx, double w, double w2, int g, const z64 (&v)[RM], const z64* vw) {
+    const int n = __builtin_amdgcn_readfirstlane(s.n), lane = threadIdx.x & 63;
+    int row[RM];
+    bool in[RM];
+#pragma unroll
+    for (int t = 0; t < RM; ++t) {
+        in[t] = lane + 64 * t < n;
+        row[t] = in[t] ? lane + 64 * t : n - 1;
+    }
+    const z64* Fg = reinterpret_cast<const z64*>(s.F) + (size_t)g * s.ldf;
+    z64 r[RM], f[RM], xv[RM];
+    double as[RM];
+#pragma unroll
+    for (int t = 0; t < RM; ++t) {
+        f[t] = ldc<1>(Fg + row[t]);
+        f[t].re = in[t] ? f[t].re : 0.0;
+        f[t].im = in[t] ? f[t].im : 0.0;
+        r[t] = f[t];
+        xv[t] = cmk<double>(in[t] ? v[t].re : 0.0, in[t] ? v[t].im : 0.0);
+        as[t] = 0.0;
+    }
+    with_kind(s, [&](auto kc) {
+        constexpr int KIND = decltype(kc)::value;
+        for (int c0 = 0; c0 < n; c0 += 4) {
+            z64 a[4][RM];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int t = 0; t < RM; ++t)
+                    a[q][t] = elem_at<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c0 + q < n) {
+                    const z64 xc = ldc<3>(vw + c0 + q);
+#pragma unroll
+                    for (int t = 0; t < RM; ++t) {
+                        as[t] += zabs(a[q][t]);
+                        cfms(r[t], a[q][t], xc);
+                    }
+                }
+        }
+    });
+    double an = 0.0;
+#pragma unroll
+    for (int t = 0; t < RM; ++t) {
+        an = nmax(an, as[t]);
+        r[t].re = in[t] ? r[t].re : 0.0;
+        r[t].im = in[t] ? r[t].im : 0.0;
+    }
+    const double be = backward_error(wave_zmax<RM>(r), wave_dmax(an), wave_zmax<RM>(xv), wave_zmax<RM>(f));
+    if (s.berr && lane == 0) s.berr[(size_t)fidx * s.nrhs + g] = be;
+}
+
+// Right-hand sides g0 .. g0 + na - 1 (na <= NW / 2, the last of the point) by every wavefront:
+// columns split over them, partial sums in LDS (part: NW (2 na + 1) n doubles, where U was).
+// One wavefront per right-hand side left the others idle for a pass over A(w) with one
+// column batch in flight (n = 128 with D, 1 right-hand side, 1024 points: 1047 us, 919 now).
+template <int NW, int RM>
+__device__ __forceinline__ void reg_berr_joint(const SysDesc& s, int fidx, double w, double w2, int g0, int na, const z64 (&v)[RM],
+                                               const z64* vec, z64* part) {
+    constexpr int NA = NW / 2;
+    const int n = __builtin_amdgcn_readfirstlane(s.n), lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double* asums = reinterpret_cast<double*>(part + (size_t)NW * na * n);  // [wavefront][n]
+    int row[RM];
+    bool in[RM];
+    z64 acc[RM][NA];
+    double as[RM];
+#pragma unroll
+    for (int t = 0; t < RM; ++t) {
+        in[t] = lane + 64 * t < n;
+        row[t] = in[t] ? lane + 64 * t : n - 1;
+        as[t] = 0.0;
+#pragma unroll
+        for (int g = 0; g < NA; ++g) acc[t][g] = czero<double>();
+    }
+    __syncthreads();  // every solution is in LDS, U is free
+    with_kind(s, [&](auto kc) {
+        constexpr int KIND = decltype(kc)::value;
+        for (int c0 = 4 * wave; c0 < n; c0 += 4 * NW) {
+            z64 a[4][RM];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int t = 0; t < RM; ++t) a[q][t] = elem_at<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c0 + q < n) {
+#pragma unroll
+                    for (int t = 0; t < RM; ++t) as[t] += zabs(a[q][t]);
+#pragma unroll
+                    for (int g = 0; g < NA; ++g)
+                        if (g < na) {
+                            const z64 x = ldc<3>(vec + (g * n + c0 + q));
+#pragma unroll
+                            for (int t = 0; t < RM; ++t) cfma(acc[t][g], a[q][t], x);
+                        }
+                }
+        }
+    });
+#pragma unroll
+    for (int t = 0; t < RM; ++t)
+        if (in[t]) {
+            asums[wave * n + row[t]] = as[t];
+#pragma unroll
+            for (int g = 0; g < NA; ++g)
+                if (g < na) stc<3>(part + ((wave * na + g) * n + row[t]), acc[t][g]);
+        }
+    __syncthreads();
+    if (wave >= na) return;
+    const z64* Fg = reinterpret_cast<const z64*>(s.F) + (size_t)(g0 + wave) * s.ldf;
+    z64 r[RM], f[RM], xv[RM];
+    double an = 0.0;
+#pragma unroll
+    for (int t = 0; t < RM; ++t) {
+        f[t] = ldc<1>(Fg + row[t]);
+        z64 a = czero<double>();
+        double sa = 0.0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            const z64 p = ldc<3>(part + ((q * na + wave) * n + row[t]));
+            a.re += p.re;
+            a.im += p.im;
+            sa += asums[q * n + row[t]];
+        }
+        an = nmax(an, sa);
+        r[t] = cmk<double>(in[t] ? f[t].re - a.re : 0.0, in[t] ? f[t].im - a.im : 0.0);
+        f[t].re = in[t] ? f[t].re : 0.0;
+        f[t].im = in[t] ? f[t].im : 0.0;
+        xv[t] = cmk<double>(in[t] ? v[t].re : 0.0, in[t] ? v[t].im : 0.0);
+    }
+    const double be = backward_error(wave_zmax<RM>(r), wave_dmax(an), wave_zmax<RM>(xv), wave_zmax<RM>(f));
+    if (s.berr && lane == 0) s.berr[(size_t)fidx * s.nrhs + g0 + wave] = be;
+}
+
 template <int NW, int RM, int CPW, bool ADJ>
 __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, const KParams& kp, char* smem) {
     constexpr int NE = 2;  // right-hand sides per wavefront and factorisation
+    constexpr int NA = NW / 2;  // up to here the backward errors are every wavefront's work
     const int n = __builtin_amdgcn_readfirstlane(sp->n), tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nrhs = __builtin_amdgcn_readfirstlane(sp->nrhs);
@@ -892,51 +1031,6 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
                         if (in[t]) stc<3>(vw + row[t], v[t]);
                     __builtin_amdgcn_wave_barrier();
                 }
-                if (want_berr) {
-                    // r = F - A(w) x by this wavefront alone, with the row sums of |A|
-                    const z64* Fg = reinterpret_cast<const z64*>(s.F) + (size_t)g * s.ldf;
-                    z64 r[RM], f[RM], xv[RM];
-                    double as[RM];
-#pragma unroll
-                    for (int t = 0; t < RM; ++t) {
-                        f[t] = ldc<1>(Fg + row[t]);
-                        f[t].re = in[t] ? f[t].re : 0.0;
-                        f[t].im = in[t] ? f[t].im : 0.0;
-                        r[t] = f[t];
-                        xv[t] = cmk<double>(in[t] ? v[t].re : 0.0, in[t] ? v[t].im : 0.0);
-                        as[t] = 0.0;
-                    }
-                    with_kind(s, [&](auto kc) {
-                        constexpr int KIND = decltype(kc)::value;
-                        for (int c0 = 0; c0 < n; c0 += 4) {
-                            z64 a[4][RM];
-#pragma unroll
-                            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                                for (int t = 0; t < RM; ++t)
-                                    a[q][t] = elem_at<KIND>(s, row[t] + min(c0 + q, n - 1) * n, w, w2);
-#pragma unroll
-                            for (int q = 0; q < 4; ++q)
-                                if (c0 + q < n) {
-                                    const z64 xc = ldc<3>(vw + c0 + q);
-#pragma unroll
-                                    for (int t = 0; t < RM; ++t) {
-                                        as[t] += zabs(a[q][t]);
-                                        cfms(r[t], a[q][t], xc);
-                                    }
-                                }
-                        }
-                    });
-                    double an = 0.0;
-#pragma unroll
-                    for (int t = 0; t < RM; ++t) {
-                        an = nmax(an, as[t]);
-                        r[t].re = in[t] ? r[t].re : 0.0;
-                        r[t].im = in[t] ? r[t].im : 0.0;
-                    }
-                    const double be = backward_error(wave_zmax<RM>(r), wave_dmax(an), wave_zmax<RM>(xv), wave_zmax<RM>(f));
-                    if (s.berr && lane == 0) s.berr[(size_t)fidx * s.nrhs + g] = be;
-                }
                 if constexpr (adj) {  // g_r = c^H x_r, J += |g_r|^2, xi += conj(g_r) x_r
                     double re = 0.0, im = 0.0;
 #pragma unroll
@@ -952,6 +1046,11 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
                     for (int t = 0; t < RM; ++t)
                         if (in[t]) cfma(xi[t], cconj(gr), v[t]);
                 }
+            }
+            if (want_berr) {
+                const int na = min(NW, gn - e * NW);
+                if (!ADJ && na <= NA && n + 1 >= NW * (2 * na + 1)) reg_berr_joint<NW, RM>(s, fidx, w, w2, g0 + e * NW, na, v, vec, R.U);
+                else if (act) reg_berr_wave<RM>(s, fidx, w, w2, g, v, vw);
             }
             if (s.C) {
                 __syncthreads();

@@ -56,3 +56,42 @@ def test_explicit_matrices_cost_little_more_than_a_sweep(handle, n):
                              lambda: handle.sweep_dev(0, f_t, F_t, X, info, None, **args)])
     assert (info == 0).all()
     assert explicit <= 1.2 * sweep, explicit / sweep
+
+
+@pytest.mark.parametrize("n,nrhs", [(100, 1), (112, 2), (128, 1), (128, 4)])
+def test_backward_errors_cost_little(handle, n, nrhs):
+    """Plain sweep with Rayleigh damping: 1.05 to 1.07 times the sweep without them
+    (every wavefront works on them), 1.21 to 1.27 (one wavefront per load)."""
+    import torch
+    nf = 1024
+    rom, rng = synth.modal_rom(n, n, 0.01, alpha=1e-4, beta=0.5)
+    handle.rom_set(0, rom.K, rom.M, rom.D, rom.eta)
+    f_t = torch.linspace(1.0, 1200.0, nf, dtype=torch.float64, device="cuda")
+    F_t = torch.from_numpy(synth.complex_normal(rng, (nrhs, n))).cuda()
+    X, info, be = _buffers(nf, n, nrhs)
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with_be, without = _best([lambda: handle.sweep_dev(0, f_t, F_t, X, info, be, stream=st.cuda_stream),
+                              lambda: handle.sweep_dev(0, f_t, F_t, X, info, None, stream=st.cuda_stream)])
+    assert (info == 0).all() and be.max() <= 1e-13
+    assert with_be <= 1.15 * without, with_be / without
+
+
+@pytest.mark.parametrize("n", [24, 37, 64, 70, 71, 72, 128])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 4, 5, 10, 17])
+def test_backward_errors_of_every_split(handle, n, nrhs):
+    """One wavefront per load or all of them, with U's room large enough for their sums or
+    not: the errors that X has."""
+    rom, rng = synth.modal_rom(n, 30 + n, 0.02, alpha=1e-4, beta=0.5)
+    handle.rom_set(0, rom.K, rom.M, rom.D, rom.eta)
+    freq = np.array([3.0, 500.0])
+    F = synth.complex_normal(rng, (n, nrhs)) * 10.0 ** rng.uniform(-3, 3, nrhs)
+    X, info, be, _ = handle.sweep(0, freq, F, mode="plain")
+    assert (info == 0).all()
+    for j, f in enumerate(freq):
+        A = synth.assemble(rom, f)
+        den = np.abs(A).sum(1).max() * np.abs(X[j]).max(0) + np.abs(F).max(0)
+        ref = np.abs(F - A @ X[j]).max(0) / den
+        # both residuals round by at most (n + 4) u of |A| |x| + |b| a row
+        assert np.abs(be[j] - ref).max() <= 2 * (n + 4) * 2.0 ** -52
+        assert be[j].max() <= n * 2.0 ** -52 + 1e-15
