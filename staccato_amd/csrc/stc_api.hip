@@ -357,12 +357,31 @@ struct LaunchCfg {
 
 constexpr int kKindReg = 4, kKindRegAdj = 5;
 
+// Whether the register panel takes a refined sweep of one or two loads (explicit matrices: one)
+// faster than reg_kernel, orders 97..128.  reg_kernel's inverse costs what LU factors and
+// several loads would, and two of its workgroups fit a CU, three of the panel's:
+// 2 C points in a round of time 1 (C CUs), 3 C in one of 1.38 (one load; explicit matrices 1.45;
+// two loads 1.47; measured 1.34..1.41, 1.42..1.50 and 1.42..1.50).  A last round that is not full
+// takes, by the workgroups on its fullest CU, half of a round, and 0.65 or 0.88 of one.
+// n = 112, one load, real: 600 points 478 against 430 us, 1024 616 and 753, 8192 4745 and
+// 4277.  More loads, and complex operators: reg_kernel is as fast or faster (three loads
+// 0.55..1.04 of the panel's time, two and explicit 0.87..1.02, complex 0.88..1.03).
+bool panel_rounds_cheaper(const SysDesc& s, long long points, int num_cu) {
+    if (s.n <= 96 || s.nrhs > (s.real_ops ? 2 : 1) || (!s.real_ops && !s.op_stride)) return false;
+    const double c = num_cu, panel[] = {0.0, 0.65, 0.88, 1.0}, regs[] = {0.0, 0.5, 1.0};
+    auto rounds = [&](int per_cu, const double* last) {
+        const double full = floor(points / (per_cu * c));
+        return full + last[(int)ceil((points - full * per_cu * c) / c)];
+    };
+    return (s.nrhs == 2 ? 1.47 : s.real_ops ? 1.38 : 1.45) * rounds(3, panel) < rounds(2, regs);
+}
+
 // Systems that reg_kernel solves in registers: every order up to 128, unless
 // the factors themselves are asked for, the adjoint is refined (it needs the
 // inverse's transpose), or a policy set for an order in that range names
 // another kernel.  Faster than the kernels it replaces at every order measured (the
-// figures are at reg_kernel); above 128 the matrix does not fit the registers of one
-// workgroup with room to work.
+// figures are at reg_kernel), but for panel_rounds_cheaper's; above 128 the matrix does not fit
+// the registers of one workgroup with room to work.
 bool use_registers(const stc_ctx* h, int maxn, int refine, int adj, int fac) {
     if (maxn > kRegMaxN || fac || (refine && adj)) return false;
     const Policy* p = nullptr;
@@ -399,8 +418,12 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
     while (maxr < r) maxr <<= 1;
     cfg->refine = refine;
     cfg->maxr = maxr;
-    const Policy pol = policy_for(h, maxn, refine);
-    if (use_registers(h, maxn, refine, adj, fac)) {
+    Policy pol = policy_for(h, maxn, refine);
+    const bool regs = use_registers(h, maxn, refine, adj, fac);
+    // slot_budget: a scratch limit holds fewer factor slots than the panel's workgroups need
+    const bool panel = regs && refine && nsys == 1 && slot_budget == 0 && panel_rounds_cheaper(sys[0], nitems, h->num_cu);
+    if (panel) pol = Policy{};
+    else if (regs) {
         cfg->wide = adj ? kKindRegAdj : kKindReg;
         cfg->threads = 64 * reg_waves(refine, maxr);
         cfg->lds = 0;
