@@ -695,8 +695,8 @@ __device__ __forceinline__ void inpanel_update(cx<T>* __restrict__ P, int m, int
 // trailing matrix per LDS panel (n = 256: 10.2 against 3.5 MB a point in complex128,
 // 4.4 of 5.2 TB/s, its bound).
 //
-// from_slot: the columns' current values are in the slot (partly updated, or
-// right-hand sides, j0 >= n), else A(w) is assembled from the operators.  Afterwards the rows
+// from_slot: the columns' current values are in the slot (partly updated), else A(w) is
+// assembled from the operators; right-hand sides (columns from n on) are in the slot.  Afterwards the rows
 // from kb1 * 16 on go to the LDS panel P (ld ldp, the first wp columns, padded with zeros
 // to a multiple of 16) and to the slot (the columns from wp on).
 // G3: Gauss 3M products (three accumulators, converted at the ends and every 32 finished
@@ -765,24 +765,25 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
         }
         if (kSB * c < wl) {
             if (c == 0 || !whole) {
-                const int nc = min(whole ? kSB * NCT : kSB, wl - kSB * c), nbat = (nc + kPB - 1) / kPB;
-                auto fill = [&](auto&& entry) {
+                const int nc = min(whole ? kSB * NCT : kSB, wl - kSB * c);
+                const int na = from_slot ? 0 : max(0, min(nc, n - j0 - kSB * c));  // assembled
+                auto fill = [&](int c0, int c1, auto&& entry) {
+                    const int nbat = (c1 - c0 + kPB - 1) / kPB;
                     for (int e = tid; e < nr * nbat; e += kThreads) {
-                        const int r = rb + e % nr, cb = e / nr * kPB;
+                        const int r = rb + e % nr, cb = c0 + e / nr * kPB;
                         const int pr = lds1<3>(rmap + r);
                         cx<T> v[kPB];
 #pragma unroll
-                        for (int u = 0; u < kPB; ++u) v[u] = entry(pr + (size_t)(j0 + kSB * c + min(cb + u, nc - 1)) * n);
+                        for (int u = 0; u < kPB; ++u) v[u] = entry(pr + (size_t)(j0 + kSB * c + min(cb + u, c1 - 1)) * n);
 #pragma unroll
                         for (int u = 0; u < kPB; ++u)
-                            if (cb + u < nc) stc<3>(P + (r + (cb + u) * ldn), v[u]);
+                            if (cb + u < c1) stc<3>(P + (r + (cb + u) * ldn), v[u]);
                     }
                 };
                 if (c) __syncthreads();
-                if (from_slot)
-                    fill([&](size_t e) { return ldc<1>(S + e); });
-                else
-                    with_kind(sd, [&](auto kc) { fill([&](size_t e) { return to_t<T>(elem_at<decltype(kc)::value>(sd, e, w, w2)); }); });
+                if (na < nc) fill(na, nc, [&](size_t e) { return ldc<1>(S + e); });
+                if (na > 0)
+                    with_kind(sd, [&](auto kc) { fill(0, na, [&](size_t e) { return to_t<T>(elem_at<decltype(kc)::value>(sd, e, w, w2)); }); });
                 __syncthreads();
             }
             const cx<T>* pt = P + (whole ? kSB * c * ldn : 0);
@@ -924,7 +925,10 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
 // ---- the wide-panel factorisation ------------------------------------------------------------
 // Left-looking in steps of 16 NCT columns (32 complex64, 16 complex128: what the
 // accumulators hold beside the operands), each step one or two LDS panels of jb columns; the
-// first group of right-hand sides last, as columns n .. n + nr - 1.
+// first group of right-hand sides last, as columns n .. n + nr - 1.  Where the last step has
+// room for them they are its columns too, and only its own blocks are left to apply
+// afterwards (a pass over all blocks for them alone made n = 129..132 plain 2 to 4 % slower than
+// right-looking panels had been: n = 129, 1 load, 1024 points 846 us, 795 now).
 template <typename T, int MAXR, bool G3>
 __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w2, cx<T>* __restrict__ S,
                                             const Layout& lay, const Lds& L, int nr) {
@@ -954,16 +958,19 @@ __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w
     if (tid == 0) L.sc[1] = 0;
     __syncthreads();
 
+    const bool fuse = nr > 0 && (n - 1) % W + 1 + nr <= W;  // room for the right-hand sides
+    int jlast = 0;                                          // the last panel's first column
     for (int j0 = 0; j0 < n + (nr > 0 ? 1 : 0);) {
         const bool rhs = j0 >= n;
         const int first = j0 / W * W;  // the step's first column
         const bool cont = !rhs && j0 > first;  // a later panel of the step
-        const int jend = rhs ? n + nr : min(first + W, n);
-        const int jbl = rhs ? 0 : min(jb, jend - j0), m = n - j0;
+        const int jend = rhs || (fuse && first + W >= n) ? n + nr : min(first + W, n);
+        const int jbl = rhs ? 0 : min(jb, min(first + W, n) - j0), m = n - j0;
         // complex64: odd leading dimension, so the columns an MFMA operand read
         // spans start in different LDS banks (complex128 elements spread already)
         const int ldp = sizeof(T) == 4 ? (m | 1) : m;
-        left_update<T, MAXR, NCT, G3>(s, w, w2, S, Lg, n, L.rmap, j0, jend - j0, cont ? (j0 - jb) / kSB : 0,
+        const int kb0 = cont ? (j0 - jb) / kSB : rhs && fuse ? jlast / kSB : 0;
+        left_update<T, MAXR, NCT, G3>(s, w, w2, S, Lg, n, L.rmap, j0, jend - j0, kb0,
                                       rhs ? (int)nblk : j0 / kSB, rhs || cont, jb >= W, P, ldp, jbl);
         __syncthreads();
         if (rhs) break;
@@ -996,6 +1003,7 @@ __device__ __forceinline__ void factor_wide(const SysDesc& s, double w, double w
             for (int c = 0; c < jbl; ++c) stc<1>(S + (pr + (size_t)(j0 + c) * n), ldc<3>(P + (r + (size_t)c * ldp)));
         }
         __syncthreads();
+        jlast = j0;
         j0 += jbl;
     }
     if (sizeof(T) == 4) {
