@@ -376,11 +376,32 @@ bool panel_rounds_cheaper(const SysDesc& s, long long points, int num_cu) {
     return (s.nrhs == 2 ? 1.47 : s.real_ops ? 1.38 : 1.45) * rounds(3, panel) < rounds(2, regs);
 }
 
+// Whether the kernels that factor once take a plain sweep of many loads faster than reg_kernel,
+// which repeats the factorisation for every 16 loads (8 up to n = 64).  Above n = 64, C points
+// of reg_kernel take, in half passes (up to 8 loads) as the unit, one a pass and 0.55 more
+// where it is full (0.75 with backward errors); the panel's 2 C points 2 (F + s nrhs), F =
+// 1.17 - 0.0023 n for the factors and s = 0.117 - 0.00036 n a load, fitted to n = 72, 96, 128
+// with 17..128 loads (within 5 %, with backward errors 10 %).  n = 128, 512 points: 16 loads
+// 0.75 of the panel's time, 17 1.18, 32 0.94, 64 1.10, 128 1.20; with backward errors 64
+// 1.29.  Up to n = 64 reg_kernel has more workgroups on a CU and is the faster one (0.4..1.0)
+// but for more than 96 loads of n <= 32 where C to 2 C points leave most of these idle
+// (n = 32, 512 points, 256 loads: 1.20).
+bool panel_passes_cheaper(const SysDesc& s, long long points, int num_cu) {
+    const double c = num_cu;
+    if (s.nrhs <= 16 || points <= num_cu) return false;
+    if (s.n <= 64) return s.n <= 32 && s.nrhs > 96 && points <= 2 * num_cu && !s.berr;
+    const int passes = (s.nrhs + 15) / 16, full = s.nrhs / 16 + (s.nrhs % 16 > 8);
+    const double regs = (passes + (s.berr ? 0.75 : 0.55) * full) * ceil(points / c);
+    const double half = points / (2 * c), part = half - floor(half);
+    const double rounds = floor(half) + (part > 0.5 ? 1.0 : part > 0.0 ? 0.8 : 0.0);
+    return 2.0 * (1.17 - 0.0023 * s.n + (0.117 - 0.00036 * s.n) * s.nrhs) * rounds < regs;
+}
+
 // Systems that reg_kernel solves in registers: every order up to 128, unless
 // the factors themselves are asked for, the adjoint is refined (it needs the
 // inverse's transpose), or a policy set for an order in that range names
 // another kernel.  Faster than the kernels it replaces at every order measured (the
-// figures are at reg_kernel), but for panel_rounds_cheaper's; above 128 the matrix does not fit
+// figures are at reg_kernel), but for the two rules above; beyond 128 the matrix does not fit
 // the registers of one workgroup with room to work.
 bool use_registers(const stc_ctx* h, int maxn, int refine, int adj, int fac) {
     if (maxn > kRegMaxN || fac || (refine && adj)) return false;
@@ -421,7 +442,8 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
     Policy pol = policy_for(h, maxn, refine);
     const bool regs = use_registers(h, maxn, refine, adj, fac);
     // slot_budget: a scratch limit holds fewer factor slots than the panel's workgroups need
-    const bool panel = regs && refine && nsys == 1 && slot_budget == 0 && panel_rounds_cheaper(sys[0], nitems, h->num_cu);
+    const bool panel = regs && !adj && nsys == 1 && slot_budget == 0 &&
+                       (refine ? panel_rounds_cheaper(sys[0], nitems, h->num_cu) : panel_passes_cheaper(sys[0], nitems, h->num_cu));
     if (panel) pol = Policy{};
     else if (regs) {
         cfg->wide = adj ? kKindRegAdj : kKindReg;
