@@ -813,7 +813,8 @@ __device__ __forceinline__ void left_update(const SysDesc& sd, double w, double 
             for (int r = 0; r < 4; ++r) {
                 const T x = cr[q][c][r], y = cy[G3 ? q : 0][c][r];
                 cr[q][c][r] = x - y;
-                ci[q][c][r] = ci[q][c][r] - x - y;
+                // an infinite real part would leave NaN: z - x
+                ci[q][c][r] = fabs(x) == T(__builtin_inf()) ? T(0) : ci[q][c][r] - x - y;
             }
         };
         if (G3)

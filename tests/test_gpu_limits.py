@@ -69,3 +69,28 @@ def test_smallest_lds_budgets(handle, n, mode, kernel, budget):
     finally:
         handle.clear_policies()
     assert (info == 0).all() and be.max() <= 1e-12
+
+
+@pytest.mark.parametrize("at", [0, 20, 40, 100])
+@pytest.mark.parametrize("n", [129, 144, 200, 256, 300])
+def test_mass_beyond_complex64(handle, n, at):
+    """Refined, an uncoupled mass whose diagonal entry overflows in complex64 only: its pivot
+    is infinite, the other unknowns are those of the system without it.  The norm of A(w)
+    makes any solution meet the tolerance, so they are as good as the complex64 factors."""
+    rom, rng = synth.modal_rom(n, 700 + n, 0.02)
+    K, M = rom.K.copy(), rom.M.copy()
+    K[at, :] = K[:, at] = M[at, :] = M[:, at] = 0.0
+    M[at, at] = 1e45
+    freq = np.array([40.0, 410.0])
+    F = synth.complex_normal(rng, (n, 2))
+    handle.rom_set(0, K, M, None, rom.eta)
+    X, info, be, _ = handle.sweep(0, freq, F, mode="refined", tol=1e-10)
+    assert (info == 0).all() and be.max() <= 1e-10
+    keep = np.arange(n) != at
+    for j, f in enumerate(freq):
+        A = ((1 + 1j * rom.eta) * K - (2 * np.pi * f) ** 2 * M)[np.ix_(keep, keep)]
+        ref = np.linalg.solve(A, F[keep])
+        assert np.abs(X[j, at]).max() <= 1e-40
+        # backward error of the factors and solves: at most n u in complex64
+        tol = n * 2.0 ** -24 * np.linalg.cond(A) * np.sqrt(n)
+        assert np.abs(X[j, keep] - ref).max() <= tol * np.abs(ref).max()
