@@ -22,11 +22,11 @@ HOST_OUT = os.path.join(OUT_DIR, "libstaccato_host.so")
 # (refine, rows per lane, panel kind) triples of sweep_kernel, one object each
 # (panel kind 0: register panel, 1: wide LDS panel, 2: wide panel with Gauss 3M
 # products, complex64 up to n = 256, 4: register-resident
-# systems, n <= 128, 5: the same with the adjoint, complex128 only); the list matches STC_INSTANCES in csrc/stc_dispatch.hip
+# systems, n <= 128, complex128 also 5: with the adjoint, 6: with backward errors); the list matches STC_INSTANCES in csrc/stc_dispatch.hip
 INSTANCES = ([(r, m, 0) for r in (0, 1) for m in (1, 2, 4, 8, 16)] +
              [(0, m, 1) for m in (2, 4, 8)] +
              [(1, m, 1) for m in (2, 4, 8, 16)] + [(1, m, 2) for m in (2, 4)] +
-             [(r, m, 4) for r in (0, 1) for m in (1, 2)] + [(0, m, 5) for m in (1, 2)])
+             [(r, m, 4) for r in (0, 1) for m in (1, 2)] + [(0, m, w) for w in (5, 6) for m in (1, 2)])
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

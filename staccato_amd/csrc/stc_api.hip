@@ -347,7 +347,7 @@ struct LaunchCfg {
     int refine = 0;
     int maxr = 1;
     int wide = 0;   // sweep_kernel<., ., wide>: 1 wide LDS panels on the blocked path, 2 with 3M products;
-                    // reg_kernel: 4, with the adjoint 5
+                    // reg_kernel: 4, with the adjoint 5, plain with backward errors 6
     int threads = kThreads;
     int lds = 0;
     int grid = 1;
@@ -355,7 +355,7 @@ struct LaunchCfg {
     size_t slot_bytes = 0;  // bytes of one factor slot (0: no blocked system)
 };
 
-constexpr int kKindReg = 4, kKindRegAdj = 5;
+constexpr int kKindReg = 4, kKindRegAdj = 5, kKindRegBerr = 6;
 
 // Whether the register panel takes a refined sweep of one or two loads (explicit matrices: one)
 // faster than reg_kernel, orders 97..128.  reg_kernel's inverse costs what LU factors and
@@ -446,7 +446,9 @@ int plan_launch(stc_ctx* h, SysDesc* sys, int nsys, long long nitems, int refine
                        (refine ? panel_rounds_cheaper(sys[0], nitems, h->num_cu) : panel_passes_cheaper(sys[0], nitems, h->num_cu));
     if (panel) pol = Policy{};
     else if (regs) {
-        cfg->wide = adj ? kKindRegAdj : kKindReg;
+        bool berr = false;
+        for (int i = 0; i < nsys; ++i) berr = berr || sys[i].berr;
+        cfg->wide = adj ? kKindRegAdj : berr && !refine ? kKindRegBerr : kKindReg;
         cfg->threads = 64 * reg_waves(refine, maxr);
         cfg->lds = 0;
         for (int i = 0; i < nsys; ++i)

@@ -8,7 +8,7 @@ namespace stc {
 // (refine, rows per lane, panel kind) triples that are built (panel kind 0:
 // register panel, 1: wide LDS panel, 2: wide panel with Gauss 3M products,
 // complex64 up to n = 256 (beyond, the third accumulator leaves no registers), 4: register-resident
-// systems, n <= 128, 5: the same with the adjoint, complex128 only); the wide-panel kernel is not built where its LDS panel
+// systems, n <= 128, complex128 also 5: with the adjoint, 6: with backward errors); the wide-panel kernel is not built where its LDS panel
 // cannot hold 16 columns (complex128 beyond n = 512) or where every system
 // fits the LDS whole (n <= 64).
 #define STC_INSTANCES(X)                                                         \
@@ -17,7 +17,7 @@ namespace stc {
     X(0, 2, 1) X(0, 4, 1) X(0, 8, 1)                                             \
     X(1, 2, 1) X(1, 4, 1) X(1, 8, 1) X(1, 16, 1)                                \
     X(1, 2, 2) X(1, 4, 2)                                                        \
-    X(0, 1, 4) X(0, 2, 4) X(1, 1, 4) X(1, 2, 4) X(0, 1, 5) X(0, 2, 5)
+    X(0, 1, 4) X(0, 2, 4) X(1, 1, 4) X(1, 2, 4) X(0, 1, 5) X(0, 2, 5) X(0, 1, 6) X(0, 2, 6)
 
 #define STC_DECL(R, M, W)                                                        \
     void* sweep_kernel_fn_##R##_##M##_##W();                                     \

@@ -13,7 +13,7 @@
 #error "STC_INST_MAXR (1, 2, 4, 8 or 16) must be defined"
 #endif
 #ifndef STC_INST_WIDE
-#error "STC_INST_WIDE (0: register panel, 1: wide panel, 2: wide panel with 3M products, 4: register-resident systems, 5: the same with the adjoint) must be defined"
+#error "STC_INST_WIDE (0: register panel, 1: wide panel, 2: wide panel with 3M products, 4: register-resident systems, 5: the same with the adjoint, 6: with backward errors) must be defined"
 #endif
 
 #define STC_CAT2(a, b, c, d) a##b##_##c##_##d
@@ -26,7 +26,7 @@ namespace stc {
 using InstT = typename std::conditional<STC_INST_REFINE != 0, float, double>::type;
 
 #if STC_INST_WIDE >= 4
-#define STC_KERNEL reg_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE == 5>
+#define STC_KERNEL reg_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE == 5, STC_INST_WIDE == 6>
 constexpr int kInstThreads = 64 * reg_waves(STC_INST_REFINE, STC_INST_MAXR);
 #else
 #define STC_KERNEL sweep_kernel<InstT, STC_INST_MAXR, STC_INST_WIDE>

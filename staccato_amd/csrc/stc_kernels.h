@@ -247,13 +247,15 @@ enum : int { kOpReal2 = 0, kOpReal3 = 1, kOpCplx = 2, kOpOne = 3 };
 __device__ __forceinline__ int op_kind(const SysDesc& s) {
     return s.real_ops ? (s.has_D ? kOpReal3 : kOpReal2) : s.op_stride && !s.has_D ? kOpOne : kOpCplx;
 }
-// f(integral_constant<kind>) for the point's kind
-template <typename F>
+// f(integral_constant<kind>) for the point's kind.  ONE: explicit matrices as a kind of their own (the
+// plain register kernel, whose loads are all in flight either way, measured 1 to 4 % slower
+// with it)
+template <bool ONE = true, typename F>
 __device__ __forceinline__ void with_kind(const SysDesc& s, F&& f) {
     const int k = op_kind(s);
     if (k == kOpReal2) f(std::integral_constant<int, kOpReal2>{});
     else if (k == kOpReal3) f(std::integral_constant<int, kOpReal3>{});
-    else if (k == kOpOne) f(std::integral_constant<int, kOpOne>{});
+    else if (ONE && k == kOpOne) f(std::integral_constant<int, ONE ? kOpOne : kOpCplx>{});
     else f(std::integral_constant<int, kOpCplx>{});
 }
 // entry k of an explicit matrix (M aliases K; eta and w are zero, so that a part that is not

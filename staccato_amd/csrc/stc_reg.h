@@ -702,14 +702,19 @@ __device__ __forceinline__ void reg_point_refined(const SysDesc* sp, int fidx, c
 // ==== complex128 LU ================================================================================
 // Triangular substitution by one wavefront, v[t] = entry lane + 64 t of the
 // vector.  BACK: unknowns n-1 .. 0, else 0 .. n-1.  at(k, i): the coefficient of
-// unknown k in equation i (only asked for i on the far side of k, clamped otherwise);
-// diag(k): the reciprocal of the diagonal.  Blocks of KB unknowns, the next
+// unknown k in equation i (used for i on the far side of k only, clamped otherwise);
+// diag(k): the reciprocal of the diagonal.  KEEP: unknowns are kept apart as they are found.  (Without,
+// those found have zero times the current unknown subtracted, which is NaN where that one
+// overflowed; the adjoint, whose sums are not finite then either way, saves the registers.)
+// Blocks of KB unknowns, the next
 // block's coefficients loaded ahead of the chain.
-template <int RM, bool BACK, bool UNIT, typename FA, typename FD>
+template <int RM, bool BACK, bool UNIT, bool KEEP = false, typename FA, typename FD>
 __device__ __forceinline__ void wave_substitute(z64 (&v)[RM], int n, FA&& at, FD&& diag) {
     constexpr int KB = RM == 1 ? 4 : 2;
     const int lane = threadIdx.x & 63;
-    z64 a[2][KB][RM], d[2][KB];
+    z64 a[2][KB][RM], d[2][KB], x[RM];
+#pragma unroll
+    for (int t = 0; t < RM; ++t) x[t] = v[t];
     auto load = [&](int k0, z64 (&la)[KB][RM], z64 (&ld)[KB]) {
 #pragma unroll
         for (int u = 0; u < KB; ++u) {
@@ -734,14 +739,18 @@ __device__ __forceinline__ void wave_substitute(z64 (&v)[RM], int n, FA&& at, FD
 #pragma unroll
             for (int t = 0; t < RM; ++t) {
                 const int i = lane + 64 * t;
-                // the result is selected, not the coefficient: zero times an unknown that
-                // overflowed would be NaN in the unknowns already found
-                const bool far = BACK ? i < k : i > k;
-                z64 f = v[t];
-                cfms(f, la[u][t], vk);
-                if (!UNIT && i == k) v[t] = vk;
-                v[t].re = far ? f.re : v[t].re;
-                v[t].im = far ? f.im : v[t].im;
+                if (KEEP) {  // entries already found are updated too, and no longer read
+                    x[t].re = i == k ? vk.re : x[t].re;
+                    x[t].im = i == k ? vk.im : x[t].im;
+                    cfms(v[t], la[u][t], vk);
+                } else {
+                    const bool far = BACK ? i < k : i > k;
+                    z64 c = la[u][t];
+                    c.re = far ? c.re : 0.0;
+                    c.im = far ? c.im : 0.0;
+                    if (!UNIT && i == k) v[t] = vk;
+                    cfms(v[t], c, vk);
+                }
             }
         }
     };
@@ -754,6 +763,9 @@ __device__ __forceinline__ void wave_substitute(z64 (&v)[RM], int n, FA&& at, FD
         load(k + 2 * KB * dir, a[0], d[0]);
         step(k + KB * dir, a[1], d[1]);
     }
+    if (KEEP)
+#pragma unroll
+        for (int t = 0; t < RM; ++t) v[t] = x[t];
 }
 
 // sum over the wavefront, in every lane
@@ -787,7 +799,7 @@ __device__ __forceinline__ void reg_berr_wave(const SysDesc& s, int fidx, double
         xv[t] = cmk<double>(in[t] ? v[t].re : 0.0, in[t] ? v[t].im : 0.0);
         as[t] = 0.0;
     }
-    with_kind(s, [&](auto kc) {
+    with_kind<false>(s, [&](auto kc) {
         constexpr int KIND = decltype(kc)::value;
         for (int c0 = 0; c0 < n; c0 += 4) {
             z64 a[4][RM];
@@ -816,7 +828,7 @@ __device__ __forceinline__ void reg_berr_wave(const SysDesc& s, int fidx, double
         r[t].im = in[t] ? r[t].im : 0.0;
     }
     const double be = backward_error(wave_zmax<RM>(r), wave_dmax(an), wave_zmax<RM>(xv), wave_zmax<RM>(f));
-    if (s.berr && lane == 0) s.berr[(size_t)fidx * s.nrhs + g] = be;
+    if (lane == 0) s.berr[(size_t)fidx * s.nrhs + g] = be;
 }
 
 // Right-hand sides g0 .. g0 + na - 1 (na <= NW / 2, the last of the point) by every wavefront:
@@ -898,10 +910,11 @@ __device__ __forceinline__ void reg_berr_joint(const SysDesc& s, int fidx, doubl
         xv[t] = cmk<double>(in[t] ? v[t].re : 0.0, in[t] ? v[t].im : 0.0);
     }
     const double be = backward_error(wave_zmax<RM>(r), wave_dmax(an), wave_zmax<RM>(xv), wave_zmax<RM>(f));
-    if (s.berr && lane == 0) s.berr[(size_t)fidx * s.nrhs + g0 + wave] = be;
+    if (lane == 0) s.berr[(size_t)fidx * s.nrhs + g0 + wave] = be;
 }
 
-template <int NW, int RM, int CPW, bool ADJ>
+// BERR: with backward errors.
+template <int NW, int RM, int CPW, bool ADJ, bool BERR>
 __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, const KParams& kp, char* smem) {
     constexpr int NE = 2;  // right-hand sides per wavefront and factorisation
     constexpr int NA = NW / 2;  // up to here the backward errors are every wavefront's work
@@ -946,7 +959,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
         {
             const SysDesc s = reg_sys(sp, fidx);
             const double w = s.freq ? kTwoPi * s.freq[fidx] : 0.0, w2 = w * w;
-            with_kind(s, [&](auto kc) {
+            with_kind<false>(s, [&](auto kc) {
                 constexpr int KIND = decltype(kc)::value;
 #pragma unroll
                 for (int qc = 0; qc < CPW; qc += 4) {
@@ -992,7 +1005,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
         const int rot = reg_eliminate<double, NW, RM, CPW, NE, false, NW == 8, ADJ>(x, b, ne, lpos, n, R);
         const SysDesc s = reg_sys(sp, fidx);
         const double w = s.freq ? kTwoPi * s.freq[fidx] : 0.0, w2 = w * w;
-        const bool want_berr = (kp.flags & kWantBerr) || s.berr != nullptr;
+        const bool want_berr = BERR && s.berr != nullptr;
         const int info = R.sc[12];
         if (info != 0) {
             reg_singular(s, fidx, info, NW * 64);
@@ -1018,7 +1031,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int t = 0; t < RM; ++t) v[t] = ldc<3>(vw + row[t]);
-                wave_substitute<RM, true, false>(v, n, u_at, u_rd);
+                wave_substitute<RM, true, false, !ADJ>(v, n, u_at, u_rd);
                 if (s.X) {
                     double2* X = s.X + (size_t)fidx * s.ldx * s.nrhs + (size_t)g * s.ldx;
 #pragma unroll
@@ -1049,7 +1062,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
             }
             if (want_berr) {
                 const int na = min(NW, gn - e * NW);
-                if (!ADJ && na <= NA && n + 1 >= NW * (2 * na + 1)) reg_berr_joint<NW, RM>(s, fidx, w, w2, g0 + e * NW, na, v, vec, R.U);
+                if (na <= NA && n + 1 >= NW * (2 * na + 1)) reg_berr_joint<NW, RM>(s, fidx, w, w2, g0 + e * NW, na, v, vec, R.U);
                 else if (act) reg_berr_wave<RM>(s, fidx, w, w2, g, v, vw);
             }
             if (s.C) {
@@ -1204,7 +1217,8 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
 // ---- the kernel ------------------------------------------------------------------------------
 // MAXR: rows per lane of the launch's largest system (1: n <= 64, 2: n <= 128).
 // ADJ: the adjoint (complex128), an instance of its own: it keeps L in registers
-// through the substitutions.
+// through the substitutions.  BERR: plain with backward errors, an instance of its own too: their
+// code costs the solves without them 1 to 4 %, the adjoint 7 to 12 %.
 //
 // Measured against the kernels it replaced there (us a call): n = 24, 32 points,
 // plain 80 -> 39 alone; n = 60, 1000 points, host arrays, plain 556 -> 271; n = 64,
@@ -1212,7 +1226,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
 // refined 438 -> 104; n = 96 complex operators, 1500 points, plain 858 -> 698;
 // n = 123, 2048 points, 4 right-hand sides, refined 1700 -> 1399; the adjoint
 // at n = 128, 2048 points 2610 -> 2259.
-template <typename T, int MAXR, bool ADJ>
+template <typename T, int MAXR, bool ADJ, bool BERR>
 __global__ void __launch_bounds__(64 * reg_waves(sizeof(T) == 4, MAXR))
     __attribute__((amdgpu_waves_per_eu(MAXR == 1 ? 4 : 2, MAXR == 1 ? 4 : 2)))
 reg_kernel(KParams kp) {
@@ -1251,12 +1265,12 @@ reg_kernel(KParams kp) {
             }
         } else {
             if constexpr (MAXR == 1) {
-                if (n <= 32) reg_point_plain<4, 1, 8, ADJ>(sp, fidx, kp, smem);
-                else reg_point_plain<4, 1, 16, ADJ>(sp, fidx, kp, smem);
+                if (n <= 32) reg_point_plain<4, 1, 8, ADJ, BERR>(sp, fidx, kp, smem);
+                else reg_point_plain<4, 1, 16, ADJ, BERR>(sp, fidx, kp, smem);
             } else {
-                if (n <= 64) reg_point_plain<8, 1, 8, ADJ>(sp, fidx, kp, smem);
-                else if (n <= 96) reg_point_plain<8, 2, 12, ADJ>(sp, fidx, kp, smem);
-                else reg_point_plain<8, 2, 16, ADJ>(sp, fidx, kp, smem);
+                if (n <= 64) reg_point_plain<8, 1, 8, ADJ, BERR>(sp, fidx, kp, smem);
+                else if (n <= 96) reg_point_plain<8, 2, 12, ADJ, BERR>(sp, fidx, kp, smem);
+                else reg_point_plain<8, 2, 16, ADJ, BERR>(sp, fidx, kp, smem);
             }
         }
         __syncthreads();
