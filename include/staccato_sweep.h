@@ -202,7 +202,8 @@ int stc_sweep_dev_noalloc(stc_handle h, int rom_id, int nfreq,
  * Factor A(2 pi freq_hz[j]) for nfreq frequencies and return the in-place
  * L\U factors (n x n, column-major, lda = n, block j at LU + j*n*n) and the
  * 1-based pivots (block j at ipiv + j*n).  mode STC_PLAIN_FP64 writes stc_z64,
- * STC_REFINED_FP32 writes stc_c32 (the factors the refined path uses).
+ * STC_REFINED_FP32 writes stc_c32 (those of the refined path above n = 128; up to there it
+ * mostly uses the inverse, pivoted alike).
  * info as above.  Host memory; synchronous. */
 int stc_getrf(stc_handle h, int rom_id, int nfreq, const double* freq_hz,
               int mode, void* LU, int* ipiv, int* info);

@@ -630,7 +630,6 @@ __global__ void load_rhs_kernel(const double2* B, int n, int nin, const double2*
     F[e] = make_double2(re, im);
 }
 
-// T (p x n, ld p) = transpose of A (n x p, ld n)
 // Sums over the frequencies of the adjoint's per-point values adj (nfreq x nq), points with
 // info > 0 left out: blockIdx.y takes one of gridDim.y consecutive slices, a block 64
 // quantities on four interleaved rows of threads, in a fixed order.
@@ -650,6 +649,7 @@ __global__ void adjoint_sum_kernel(const double* adj, const int* info, int nfreq
         sums[(size_t)blockIdx.y * nq + k] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
 }
 
+// T (p x n, ld p) = transpose of A (n x p, ld n)
 __global__ void transpose_kernel(const double* A, int n, int p, double* T) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e < n * p) T[e] = A[e / p + (size_t)(e % p) * n];

@@ -1,21 +1,22 @@
 // stc_kernels.h -- gfx950 kernels of the frequency sweep.
 //
-// One workgroup (256 lanes = 4 wavefronts) owns one point (system, frequency)
-// at a time and takes points from a device work queue until it is empty
-// (persistent launch).  Per point it
+// One workgroup (four wavefronts, eight where one workgroup fits a CU: sweep_threads) owns one
+// point (system, frequency) at a time and takes points from a device work queue until it is
+// empty (persistent launch).  Per point it
 //   1. assembles A(w) = (1 + i eta) K + i w D - w^2 M in FP64 from the ROM
 //      operators (KrylovROMSubstructure.cpp:1412-1420) and rounds it to the
 //      factor type T (double: plain path, float: refined path),
 //   2. factors P A = L U with partial pivoting, LAPACK zgetrf semantics
 //      (KrylovROMSubstructure.cpp:1428): pivot = first row of largest
 //      |re| + |im|, full-row interchanges, unit-lower L and U in place,
+//      - orders up to 128 mostly run in registers instead (stc_reg.h);
 //      - small n: the whole matrix lives in LDS, unblocked right-looking;
 //      - larger n: the matrix lives in a per-workgroup slot of global memory
 //        (reused point after point; its traffic goes through L2 and, once the
-//        resident slots exceed the caches, HBM) and is factored blocked
-//        right-looking: a panel of jb columns (registers, or LDS in the wide
-//        path of stc_wide.h), deferred row interchanges, U12 = L11^{-1} A12
-//        and the trailing update A22 -= L21 U12 per chunk of columns,
+//        resident slots exceed the caches, HBM) and is factored blocked: left-looking
+//        with LDS panels (stc_wide.h), or right-looking with a register panel of jb
+//        columns, deferred row interchanges, U12 = L11^{-1} A12 and the trailing update
+//        A22 -= L21 U12 per chunk of columns,
 //   3. solves for all right-hand sides (KrylovROMSubstructure.cpp:1430),
 //   4. optionally refines in FP64: r = F - A x with A re-assembled in FP64,
 //      A d = r with the T factors, x += d, until the normwise backward error

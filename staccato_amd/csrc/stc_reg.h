@@ -1122,7 +1122,7 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
             }
             __syncthreads();
             // ---- nu^H K xi: rows over the lanes, columns over the wavefronts
-            double er = 0.0, ei = 0.0;
+            double ei = 0.0;
             {
                 z64 kx[RM];
 #pragma unroll
@@ -1147,12 +1147,9 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
 #pragma unroll
                 for (int t = 0; t < RM; ++t)
                     if (in[t]) {
-                        const z64 m = cmul(cconj(ldc<3>(nu + row[t])), kx[t]);
-                        er += m.re;
-                        ei += m.im;
+                        ei += cmul(cconj(ldc<3>(nu + row[t])), kx[t]).im;
                     }
             }
-            (void)er;
             ei = wave_dsum(ei);
             if (lane == 0) red[NW + wave] = ei;
             // ---- the modal products phi_k^T nu and phi_k^T xi: k over the lanes (64 at a
@@ -1268,7 +1265,7 @@ reg_kernel(KParams kp) {
                 if (n <= 32) reg_point_plain<4, 1, 8, ADJ, BERR>(sp, fidx, kp, smem);
                 else reg_point_plain<4, 1, 16, ADJ, BERR>(sp, fidx, kp, smem);
             } else {
-                if (n <= 64) reg_point_plain<8, 1, 8, ADJ, BERR>(sp, fidx, kp, smem);
+                if (!ADJ && n <= 64) reg_point_plain<8, 1, 8, false, BERR>(sp, fidx, kp, smem);  // in a batch
                 else if (n <= 96) reg_point_plain<8, 2, 12, ADJ, BERR>(sp, fidx, kp, smem);
                 else reg_point_plain<8, 2, 16, ADJ, BERR>(sp, fidx, kp, smem);
             }

@@ -180,7 +180,8 @@ __device__ __forceinline__ void subpanel_moves(cx<T>* __restrict__ P, int ldp, i
     const int nother = jbl - sbw;  // panel columns outside the sub-panel
     const int per = nother + 1;    // + the row-map entry
     const int total = cnt * per;
-    constexpr int kMv = 8;         // cnt <= 2 sbw = 32, per <= 49: <= 1568 = 6.1 per lane
+    // cnt <= 2 sbw <= 32, and beside a sub-panel lies at most the rest of the widest panel
+    constexpr int kMv = (2 * kSB * (wide_jb_max((int)sizeof(cx<T>)) - kSB + 1) + kThreads - 1) / kThreads;
     cx<T> tv[kMv];
     int ti[kMv];
 #pragma unroll
@@ -218,11 +219,11 @@ __device__ __forceinline__ void subpanel_moves(cx<T>* __restrict__ P, int ldp, i
 // ---- 16-column sub-panel of the LDS panel ------------------------------------------------
 // Columns [c0, c0 + sbw) of P (m x jb, ld m, logical row order), rows
 // [c0, m).  Every thread holds whole rows of the sub-panel (rows
-// tid + 256 t) in registers, x[c] = column c.
+// tid + kThreads t) in registers, x[c] = column c.
 // Per column one barrier: each wave finds its best candidate row (packed
 // keys, DPP), the winning lane publishes that row's 16 values and the wave's
 // key in one of two alternating LDS buffers; after the barrier every thread
-// picks the best of the four candidates (the same in all), takes the pivot
+// picks the best of the wavefronts' candidates (the same in all), takes the pivot
 // row from LDS, scales its own rows' multipliers and applies the rank-1
 // update.  Rows stay in their registers; pivots only change their logical
 // positions lpos.  Afterwards the sub-panel is stored at its new rows and the
@@ -238,7 +239,7 @@ __device__ __forceinline__ void subpanel_factor(cx<T>* __restrict__ P, int m, in
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int mq = m - c0;
     cx<T>* Q = P + c0 + (size_t)c0 * ldp;  // sub-panel origin, ld ldp
-    // candidate keys after the row buffers: 2 buffers x 4 waves x {key lo, key hi, lo, -}
+    // candidate keys after the row buffers: 2 buffers x kWaves x {key lo, key hi, lo, -}
     unsigned* cand = reinterpret_cast<unsigned*>(rowbuf + 2 * kWaves * kSB);
     cx<T> x[kSB][RM];
     int lpos[RM];
@@ -388,7 +389,7 @@ __device__ __forceinline__ void subpanel_factor(cx<T>* __restrict__ P, int m, in
                 }
             }
             __syncthreads();
-            // ---- the pivot: best of the four waves' candidates
+            // ---- the pivot: best of the wavefronts' candidates
             unsigned long long bk = 0;
             unsigned bl = 0;
             int bw = 0;
@@ -586,7 +587,7 @@ __device__ __forceinline__ void subpanel_factor_1w(cx<float>* __restrict__ P, in
 
 // ---- inverse of a unit-lower 16 x 16 diagonal block ----------------------------------------
 // From Q (LDS, ld ldq; kb <= 16 valid rows/columns), by forward substitution
-// X[i][c] -= L[i][k] X[k][c] (i > k) over all 256 threads, one entry each;
+// X[i][c] -= L[i][k] X[k][c] (i > k) over 256 threads, one entry each;
 // X[k][c] comes from the same wavefront by one cross-lane read per part.
 // Linv (LDS, 16 x 16, ld 16) is zero outside the kb x kb block; Lg (slot,
 // ld kb) gets the kb x kb block for the triangular solves.
