@@ -39,8 +39,8 @@ PEAK_HBM_GBS = 8000.0
 # bytes copied: x2.0; WRITE_SIZE reads them exactly: x1.0).  The summary and the
 # commands are in profiles/sweep_kernel_n256_left_looking.txt; re-measure when the kernel changes.
 TRAFFIC_KIB = {
-    ("refined", "wide-3M-2perCU"): (6.186e6, 3.044e6),
-    ("plain", "wide-2perCU"): (16.52e6, 5.100e6),
+    ("refined", "wide-3M-2perCU"): (6.022e6, 3.032e6),
+    ("plain", "wide-2perCU"): (16.34e6, 5.091e6),
 }
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
 

@@ -1218,11 +1218,11 @@ __device__ __forceinline__ void reg_point_plain(const SysDesc* sp, int fidx, con
 // code costs the solves without them 1 to 4 %, the adjoint 7 to 12 %.
 //
 // Measured against the kernels it replaced there (us a call): n = 24, 32 points,
-// plain 80 -> 39 alone; n = 60, 1000 points, host arrays, plain 556 -> 271; n = 64,
-// 4096 explicit matrices 1708 -> 465; n = 47, 1501 points, 2 right-hand sides,
-// refined 438 -> 104; n = 96 complex operators, 1500 points, plain 858 -> 698;
-// n = 123, 2048 points, 4 right-hand sides, refined 1700 -> 1399; the adjoint
-// at n = 128, 2048 points 2610 -> 2259.
+// plain 80 -> 39 alone; n = 60, 1000 points, host arrays, plain 557 -> 195 (76 of it by
+// the results' way back); n = 64, 4096 explicit matrices 1708 -> 471; n = 47, 1501
+// points, 2 right-hand sides, refined 437 -> 103; n = 96 complex operators, 1500
+// points, plain 831 -> 677; n = 123, 2048 points, 4 right-hand sides, refined
+// 1698 -> 1381; the adjoint at n = 128, 2048 points 2627 -> 1900.
 template <typename T, int MAXR, bool ADJ, bool BERR>
 __global__ void __launch_bounds__(64 * reg_waves(sizeof(T) == 4, MAXR))
     __attribute__((amdgpu_waves_per_eu(MAXR == 1 ? 4 : 2, MAXR == 1 ? 4 : 2)))
